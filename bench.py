@@ -575,8 +575,9 @@ GENERAL_SHAPES = (
 def general_bench(length: int, steps: int, warmup: int) -> dict:
     """The general attention kernel (faq_attention_fwd_general: key tiles and head dims the
     MFMA kernel does not take, fp32 operands) on Qwen3-8B heads (32 query / 8 KV heads),
-    causal prefill over `length` tokens, HIP events around `steps` launches.  The kernel
-    multiplies in fp32 on the VALU; its roofline is MI355X's fp32 peak (157.3 TFLOP/s)."""
+    causal prefill over `length` tokens, HIP events around `steps` launches.  The rate is also
+    given against MI355X's fp32 matrix peak (157.3 TFLOP/s), which bounds the fp32 shape; 16-bit
+    operands run on their own, faster matrix instructions."""
     import torch
 
     from faquant_amd import _ops

@@ -20,6 +20,9 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "faquant_amd", "libfaquant_amd.so")
 ATTN_MASK_FORMS = 5  # attn_instances.hip is compiled once per masking form
+# attn_generic.hip is compiled once per operand form (its MFMA types, 10 * scores + PV) and
+# once for the launcher
+GENERAL_FORMS = ("00", "02", "10", "12", "20", "22")
 
 COMPILE = [
     "--offload-arch=gfx950",
@@ -49,12 +52,15 @@ def _run(cmd: list[str], verbose: bool) -> None:
 
 def build(verbose: bool = False) -> str:
     """Compile the C ABI, the decode kernels and the attention instantiations (one object
-    per masking form), in parallel, and link libfaquant_amd.so."""
+    per masking form or operand form), in parallel, and link libfaquant_amd.so."""
     with tempfile.TemporaryDirectory(prefix="faq_build_") as tmp:
         units = [(os.path.join(CSRC, "capi.hip"), [], os.path.join(tmp, "capi.o")),
                  (os.path.join(CSRC, "attn_decode.hip"), [], os.path.join(tmp, "attn_decode.o")),
                  (os.path.join(CSRC, "hif4_linear.hip"), [], os.path.join(tmp, "hif4_linear.o")),
                  (os.path.join(CSRC, "attn_generic.hip"), [], os.path.join(tmp, "attn_generic.o"))]
+        for f in GENERAL_FORMS:
+            units.append((os.path.join(CSRC, "attn_generic.hip"), [f"-DFAQ_GEN_FORM={f}"],
+                          os.path.join(tmp, f"attn_g{f}.o")))
         for m in range(ATTN_MASK_FORMS):
             units.append((os.path.join(CSRC, "attn_instances.hip"), [f"-DFAQ_ATTN_MASK={m}"],
                           os.path.join(tmp, f"attn_m{m}.o")))

@@ -1,5 +1,5 @@
 // General-shape HiF4 attention (any head_dim up to 256, any key tile up to 1024, fp32, bf16
-// or fp16 operands multiplied in fp32): arguments and launcher.
+// or fp16 operands): arguments and launcher.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -7,10 +7,8 @@
 
 namespace faq {
 
-constexpr int kGenRows = 16;         // query rows per workgroup
 constexpr int kGenMaxDim = 256;      // head_dim limit
 constexpr int kGenMaxTile = 1024;    // key tile limit
-constexpr int kGenChunk = 32;        // keys staged in LDS at a time
 
 struct GenAttnArgs {
   // operands [B, H, L, D] at element strides (last stride 1); dtype 0 fp32, 1 bf16, 2 fp16
@@ -30,6 +28,7 @@ struct GenAttnArgs {
   int causal;
   float scale;
   float softcap;  // > 0: scores -> softcap tanh(scores / softcap) after the scale
+  float softcap_rec;  // fp32(1 / softcap)
   int quant_p;    // HiF4 QDQ of P per 64-key group of each key tile
   int p_levels;
   int norm_same;  // the normalizer sums P^ (quantized_same) instead of P
@@ -44,12 +43,19 @@ struct GenAttnArgs {
   const float* amask;
   int64_t am_sb, am_sh, am_sq;
   float* diag;  // PV-normalizer probe sums per row, [B, Hq, Lq, 5] (needs quant_p)
+  // set by the launcher: query heads per workgroup and position blocks per head group
+  int hpw, n_pblocks;
 };
 
-// Dynamic LDS bytes of one workgroup for head_dim D and key tile T.
-size_t gen_attention_lds_bytes(int D, int T);
+// Workgroups of one batch entry (grid x), or -1 if they do not fit a grid.
+int64_t gen_attention_blocks(const GenAttnArgs& a);
 
-// hipSuccess, or the error of raising the kernel's dynamic LDS limit (nothing launched).
-hipError_t launch_gen_attention(const GenAttnArgs& a, hipStream_t st);
+// a.B <= 65535 and gen_attention_blocks(a) >= 0
+void launch_gen_attention(const GenAttnArgs& a, hipStream_t st);
+
+// One object per operand form (attn_generic.hip): kQK the scores' MFMA (0 bf16, 1 fp16,
+// 2 fp32), kPV the PV product's (0 bf16, 2 fp32).
+template <int kQK, int kPV>
+void launch_gen_form(const GenAttnArgs& a, dim3 grid, hipStream_t st);
 
 }  // namespace faq

@@ -1036,6 +1036,7 @@ int faq_attention_fwd_general(const void* q, int q_dtype, int64_t q_sb, int64_t 
     if (opts->p_dump || opts->q_prep) return fail(FAQ_EUNSUP, "%s: p_dump and q_prep are options of faq_attention_fwd", who);
     if (opts->softcap < 0.0f || !(opts->softcap == opts->softcap)) return fail(FAQ_EINVAL, "%s: bad softcap", who);
     a.softcap = opts->softcap;
+    a.softcap_rec = a.softcap > 0.0f ? 1.0f / a.softcap : 0.0f;
     const bool any_range = opts->row_lo || opts->row_hi || opts->key_bits;
     if (any_range && !(opts->row_lo && opts->row_hi && opts->key_bits))
       return fail(FAQ_EINVAL, "%s: row_lo, row_hi and key_bits go together", who);
@@ -1053,12 +1054,8 @@ int faq_attention_fwd_general(const void* q, int q_dtype, int64_t q_sb, int64_t 
     if (opts->pv_probe && !quant_p) return fail(FAQ_EINVAL, "%s: pv_probe needs quant_p", who);
     a.diag = opts->pv_probe;
   }
-  const hipError_t e = faq::launch_gen_attention(a, static_cast<hipStream_t>(stream));
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    return fail(FAQ_ELAUNCH, "%s: LDS limit of %zu bytes refused: %s", who, faq::gen_attention_lds_bytes(D, key_tile),
-                hipGetErrorString(e));
-  }
+  if (faq::gen_attention_blocks(a) < 0) return fail(FAQ_EUNSUP, "%s: too many work items", who);
+  faq::launch_gen_attention(a, static_cast<hipStream_t>(stream));
   return check_launch(who);
 }
 

@@ -443,6 +443,9 @@ def general_attend(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, 
         _ops.attention_fwd(bf(q_op), bf(k_op), transposed_values(bf(v_op)), key.shape[2], quant_p=pv_quant,
                            p_levels=levels["p"], out=out32, **attn)
         return out.copy_(out32[..., :D])
+    # quantized operands as bf16 (exact, see above): the kernel multiplies them on the bf16 MFMA
+    q_op, k_op = (t.to(torch.bfloat16) if qk_quant else t for t in (q_op, k_op))
+    v_op = v_op.to(torch.bfloat16) if pv_quant else v_op
     return _ops.attention_general(q_op, k_op, v_op, key_tile=key_chunk, quant_p=pv_quant, p_levels=levels["p"],
                                   out=out, **attn)
 
