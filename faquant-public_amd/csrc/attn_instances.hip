@@ -13,13 +13,21 @@ namespace {
 template <int LV, int kMask>
 void launch_lv(const AttnArgs& a, int quant_p, int same, dim3 grid, hipStream_t st) {
   if (a.diag || a.p_dump) {  // the probe form exists only with P quantization (validated by the caller)
-    if (same) hipLaunchKernelGGL((attn_fwd_kernel<LV, true, true, kMask | 8>), grid, dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((attn_fwd_kernel<LV, true, false, kMask | 8>), grid, dim3(512), 0, st, a);
+    if (same) hipLaunchKernelGGL((attn_fwd_kernel<LV, true, true, kMask | 8, 8>), grid, dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((attn_fwd_kernel<LV, true, false, kMask | 8, 8>), grid, dim3(512), 0, st, a);
     return;
   }
-  if (quant_p && same) hipLaunchKernelGGL((attn_fwd_kernel<LV, true, true, kMask>), grid, dim3(512), 0, st, a);
-  else if (quant_p) hipLaunchKernelGGL((attn_fwd_kernel<LV, true, false, kMask>), grid, dim3(512), 0, st, a);
-  else hipLaunchKernelGGL((attn_fwd_kernel<LV, false, false, kMask>), grid, dim3(512), 0, st, a);
+  if constexpr (attn_four_waves(kMask)) {
+    if (a.waves == 4) {
+      if (quant_p && same) hipLaunchKernelGGL((attn_fwd_kernel<LV, true, true, kMask, 4>), grid, dim3(256), 0, st, a);
+      else if (quant_p) hipLaunchKernelGGL((attn_fwd_kernel<LV, true, false, kMask, 4>), grid, dim3(256), 0, st, a);
+      else hipLaunchKernelGGL((attn_fwd_kernel<LV, false, false, kMask, 4>), grid, dim3(256), 0, st, a);
+      return;
+    }
+  }
+  if (quant_p && same) hipLaunchKernelGGL((attn_fwd_kernel<LV, true, true, kMask, 8>), grid, dim3(512), 0, st, a);
+  else if (quant_p) hipLaunchKernelGGL((attn_fwd_kernel<LV, true, false, kMask, 8>), grid, dim3(512), 0, st, a);
+  else hipLaunchKernelGGL((attn_fwd_kernel<LV, false, false, kMask, 8>), grid, dim3(512), 0, st, a);
 }
 
 }  // namespace

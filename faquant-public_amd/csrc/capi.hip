@@ -156,8 +156,8 @@ int device_cus() {
 
 // Workgroups of the attention kernel for n_items work items per split: one per CU in total
 // (a multiple of 8 when that many), never more than the items.
-int workers_for(int n_items, int nsplit) {
-  int p = std::max(1, device_cus() / std::max(1, nsplit));
+int workers_for(int n_items, int nsplit, int per_cu = 1) {
+  int p = std::max(1, per_cu * device_cus() / std::max(1, nsplit));
   if (p >= 8) p -= p % 8;
   return std::max(1, std::min(n_items, p));
 }
@@ -287,6 +287,7 @@ int attention_setup(const char* who, const uint16_t* q, int64_t q_sb, int64_t q_
   // the softcap and dense-mask paths scale the scores themselves, which then enter the
   // exponent unscaled
   a.c1 = static_cast<float>(static_cast<double>(a.softcap > 0.0f || a.amask ? 1.0f : scale) * 1.4426950408889634);
+  a.waves = 8;
   a.hpw = hpw;
   a.n_pblocks = (Lq + pos_per_wg - 1) / pos_per_wg;
   a.row_den = row_den;
@@ -306,6 +307,31 @@ void launch_attention(const faq::AttnArgs& a, int quant_p, int p_levels, int nor
   else if (a.softcap > 0.0f) faq::launch_attention_mask<2>(a, quant_p, p_levels, norm_same, grid, st);
   else if (a.row_lo) faq::launch_attention_mask<1>(a, quant_p, p_levels, norm_same, grid, st);
   else faq::launch_attention_mask<0>(a, quant_p, p_levels, norm_same, grid, st);
+}
+
+// Whether a launch of n_items eight-wave work items runs as four-wave workgroups instead, two
+// per CU.  Eight waves share each K/V tile among 256 rows (half the LDS traffic) and win by
+// 2-5% where every CU has several long items; four waves win where the longest item decides
+// (one wave per SIMD takes 0.6 of two waves' time per tile, and a CU's pair is a long and a
+// short item) and where items are short (one workgroup's setup and epilogue run under the
+// other's tiles).  Measured on 256 CUs, eight against four waves, us:
+//   causal, up to 1.4 items per CU: 32/8 heads 1024 tokens 47.5 / 35.1, 2048 80.3 / 62.4, 2600
+//     99.8 / 86.8, 512 of 8704 keys 284 / 206; just above: 3400 tokens 125 / 127, 4096 164 / 170
+//   causal, many short items: 16 x 512 107 / 99, 8 x 700 81.4 / 77.0; 16 x 1024 269 / 270;
+//     long ones: 8192 tokens 604 / 627
+//   key ranges (items of unequal length): 4 x 1000 64.5 / 53.1, 8 x 1500 193 / 182, 4 x 8000
+//     1552 / 1536; 2 x 16000 3927 / 4084
+//   not causal: 40 heads, 5000 of 640 keys 134 / 131, 20000 of 257 346 / 336; of 2048 240 / 244;
+//     one equal item per CU at most: 1500 tokens 67.3 / 68.8
+bool four_waves(const faq::AttnArgs& a, int64_t n_items) {
+  if (a.diag || a.p_dump || a.amask || a.softcap > 0.0f) return false;  // eight-wave forms only
+  const char* env = std::getenv("FAQ_ATTN_WAVES");  // test hook: 4 or 8
+  if (env && (env[0] == '4' || env[0] == '8')) return env[0] == '4';
+  const int64_t cus = device_cus();
+  if (a.row_lo) return a.Lk <= 8192;
+  if (!a.causal) return 2 * n_items <= cus || (n_items > cus && a.Lk <= 1024);
+  const int64_t mean_keys = a.Lk - a.Lq / 2;  // keys seen by a row, on average
+  return 5 * n_items <= 7 * cus || (n_items > 2 * cus && mean_keys <= 512);
 }
 
 int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
@@ -699,6 +725,16 @@ int faq_attention_fwd(const uint16_t* q, int64_t q_sb, int64_t q_sh, int64_t q_s
     a.pace_epoch = e;
     const char* lead_env = std::getenv("FAQ_ATTN_PACE_LEAD");  // test hook: the lead in tiles
     a.pace_lead = lead_env ? std::max(1, std::atoi(lead_env)) : faq::kPaceLead;
+  }
+  if (four_waves(a, n_items_of(a))) {
+    a.waves = 4;
+    a.cus8 = std::max(1, device_cus() / 8);
+    a.hpw = std::min(a.hpw, 4);
+    const int pos = 32 * (4 / a.hpw);
+    a.n_pblocks = (Lq + pos - 1) / pos;
+    const int64_t n_items = static_cast<int64_t>(B) * (Hq / a.hpw) * a.n_pblocks;
+    if (n_items > INT32_MAX) return fail(FAQ_EUNSUP, "faq_attention_fwd: too many work items");
+    grid.x = static_cast<unsigned>(workers_for(static_cast<int>(n_items), 1, 2));
   }
   launch_attention(a, quant_p, p_levels, norm_same, grid, static_cast<hipStream_t>(stream));
   return check_launch("faq_attention_fwd");

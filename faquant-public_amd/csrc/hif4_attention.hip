@@ -20,6 +20,13 @@
 // DMA of tile t + 1 (or of the next item's first tile) is issued at the top of tile t,
 // behind the tile's single barrier.
 //
+// Four-wave form (kW = 4): 128 rows per item, 256 threads and one LDS stage (68 KiB), so two
+// workgroups run on each CU, one wave of each per SIMD.  K tile t + 1 is loaded into the K
+// half once every wave has its scores of tile t (a second barrier per tile), V^T tile t into
+// the V half at the top of tile t, under QK and the row maximum.  The same operations in the
+// same order on every row, so the same bits; capi.hip (four_waves) says which launches take it
+// and what both forms measured.
+//
 // Masks: bottom-right causal from the shapes, or per-row key ranges [row_lo, row_hi]
 // plus a key-validity bitmap (2-D padding masks in the unpadded-rank form of sfa:371-427,
 // sliding windows), or a dense additive fp32 mask (3-D/4-D masks, sfa:430-454); keys
@@ -77,6 +84,8 @@ struct AttnArgs {
   int B, Hq, Hkv, Lq, Lk;
   int causal;
   float c1;  // softmax scale * log2(e)
+  int cus8;       // CUs / 8 (the four-wave form's pairing)
+  int waves;      // waves of 32 query rows per workgroup: 8 (one workgroup per CU) or 4 (two)
   int hpw;        // query heads per workgroup: 1, 2, 4 or 8
   int n_pblocks;  // position blocks per head group
   float* row_den;  // optional fp32 [B, Hq, Lq]: final denominator l
@@ -150,6 +159,9 @@ static __device__ uint32_t attn_pace[kPaceEpochs * 8];
 __device__ __forceinline__ bool pace_ahead(int step, uint32_t seen, int nw, int lead) {
   return static_cast<int32_t>(static_cast<uint32_t>(step * nw) - seen - static_cast<uint32_t>(lead * nw)) > 0;
 }
+
+// Masking forms (kMask) whose kernel exists with four waves per workgroup.
+constexpr bool attn_four_waves(int mask) { return mask == 0 || mask == 1; }
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void lds_void;
@@ -581,6 +593,7 @@ constexpr int kTileBytes = kKeyTile * kRowUnits * 16;  // 34816
 constexpr int kStageBytes = 2 * kTileBytes;             // K tile, then V^T tile
 constexpr int kOutPitch = 136;  // bf16 elements per staged output row (272 B): 8 waves x 32 rows fit one stage
 static_assert(8 * 32 * kOutPitch * 2 <= kStageBytes, "staged output rows must fit one LDS stage");
+static_assert(4 * 32 * kOutPitch * 2 <= kTileBytes, "and four waves' rows the V^T tile");
 
 __device__ __forceinline__ bf16x8 lds_read_at(const uint8_t* base, int byte_off) {
   return *reinterpret_cast<const bf16x8*>(base + byte_off);
@@ -600,16 +613,17 @@ __device__ __forceinline__ bf16x8 lds_read_at(const uint8_t* base, int byte_off)
 // one stream of key tiles: the DMA of the next item's first tile is issued during the
 // current item's last tile, and no workgroup is relaunched between items.  P = n_items
 // gives one item per workgroup.
-template <int LV, bool kQuantP, bool kSame, int kMode>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <int LV, bool kQuantP, bool kSame, int kMode, int kW>
+__global__ __launch_bounds__(64 * kW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_fwd_kernel(AttnArgs a) {
+  constexpr int kT = 64 * kW;  // threads
   constexpr int kMask = kMode & 7;
   constexpr bool kDiag = kQuantP && (kMode & 8) != 0;
   constexpr bool kDense = kMask == 3 || kMask == 4;
   constexpr bool kSoftcap = kMask == 2 || kMask == 4;
   constexpr bool kRanges = kMask == 1 || kMask == 2;
   constexpr bool kExactArg = !(kQuantP && kSame);  // see p_arg
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * kStageBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[(kW == 8 ? 2 : 1) * kStageBytes];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -621,7 +635,7 @@ void attn_fwd_kernel(AttnArgs a) {
   const int hgroups = G / a.hpw;
   const int X = a.B * a.Hkv * hgroups;
   const int n_items = X * a.n_pblocks;
-  const int pos_per_wg = 32 * (8 / a.hpw);
+  const int pos_per_wg = 32 * (kW / a.hpw);
   const int off = a.Lk - a.Lq;  // bottom-right alignment: row p sees keys <= p + off
   const int split = static_cast<int>(blockIdx.z);
   const int P = static_cast<int>(gridDim.x);
@@ -639,8 +653,13 @@ void attn_fwd_kernel(AttnArgs a) {
   // item of round k for this workgroup (n_items or more: none)
   auto item_of = [&](int k) -> int {
     if (head_major) return k * P + (wid % 8) * (P / 8) + wid / 8;
-    const int r = (k & 1) ? ((P % 8 == 0) ? (wid % 8) + 8 * (P / 8 - 1 - wid / 8) : P - 1 - wid) : wid;
-    return k * P + r;
+    if (P % 8) return k * P + ((k & 1) ? P - 1 - wid : wid);
+    int q = wid / 8;
+    // four waves: workgroups wid and wid + (number of CUs) share a CU, so the second ones run in
+    // reverse and the long items of a CU's pair meet short ones
+    if (kW == 4 && q >= a.cus8) q = a.cus8 + P / 8 - 1 - q;
+    if (k & 1) q = P / 8 - 1 - q;
+    return k * P + wid % 8 + 8 * q;
   };
   // workgroup-uniform geometry of an item: coordinates and its key-tile range
   struct Geo {
@@ -683,55 +702,75 @@ void attn_fwd_kernel(AttnArgs a) {
     __builtin_memcpy(&ones2, &one2, 4);
   }
 
-  // DMA assignment: instruction j (0..3) of wave w fills tile units 512 j + 64 w + lane;
-  // waves 0 and 1 also fill units 2048 + 64 w + lane (j = 4).  Unit u is piece u % 17 of
-  // row u / 17; the padding piece re-reads piece 15 of its row.
+  // DMA assignment, units of 16 bytes: LDS unit u is piece u % 17 of row u / 17; the padding
+  // piece re-reads piece 15 of its row.  The kHalves parts of a tile (128 / kHalves rows) are
+  // loaded alike, row offsets moved by a scalar: instruction j (0..3) of wave w fills units
+  // 64 (kW j + w) + lane of a part, and the part's last units (64 or 128 of its 2176 / kHalves)
+  // go to waves 0 (and 1) as j = 4.
   const int ws = __builtin_amdgcn_readfirstlane(w);
-  const int nj = ws < 2 ? 5 : 4;
+  constexpr int kHalves = 8 / kW;
+  constexpr int kPartRows = kKeyTile / kHalves;
+  const int nj = ws < 2 / kHalves ? 5 : 4;
   uint32_t kvo[5], vvo[5];
-  int krow[5];
 #pragma unroll
   for (int j = 0; j < 5; ++j) {
-    const int u = (j < 4 ? 512 * j : 2048) + 64 * ws + lane;
+    const int u = 64 * (kW * j + ws) + lane;
     const int r = u / kRowUnits;
     const int p = min(u - r * kRowUnits, 15);
-    krow[j] = r;
     kvo[j] = static_cast<uint32_t>(r * static_cast<int>(a.k_sl) + 8 * p) * 2u;
     vvo[j] = static_cast<uint32_t>(r * static_cast<int>(a.v_sd) + 8 * p) * 2u;
   }
   const uint32_t k_bytes = a.Lk > 0 ? static_cast<uint32_t>(((a.Lk - 1) * a.k_sl + kDim) * 2) : 0u;
   const uint32_t v_bytes = static_cast<uint32_t>((127 * a.v_sd + a.v_sd) * 2);
+  auto dma_dst = [&](uint8_t* st, int h, int j) {
+    return reinterpret_cast<uint16_t*>(st + (kPartRows * kRowUnits * h + 64 * (kW * j + ws)) * 16);
+  };
 
-  // DMA of key tile t of the item at (b, kvh) into LDS stage `stage`
-  auto load_tile = [&](int gb, int gkvh, int t, int stage) {
+  // DMA of K tile t of the item at (b, kvh) to LDS `st`
+  auto load_k = [&](int gb, int gkvh, int t, uint8_t* st) {
     const __amdgpu_buffer_rsrc_t krs = make_rsrc(a.k + gb * a.k_sb + gkvh * a.k_sh, k_bytes);
-    const __amdgpu_buffer_rsrc_t vrs = make_rsrc(a.vt + gb * a.v_sb + gkvh * a.v_sh, v_bytes);
-    uint8_t* const st = lds + stage * kStageBytes;
     const int key0 = t * kKeyTile;
-    const uint32_t ksoff = static_cast<uint32_t>(key0 * a.k_sl) * 2u;
-    const uint32_t vsoff = static_cast<uint32_t>(key0) * 2u;
-    if (key0 + kKeyTile <= a.Lk) {
 #pragma unroll
-      for (int j = 0; j < 5; ++j)
-        if (j < nj) dma16(krs, kvo[j], ksoff, reinterpret_cast<uint16_t*>(st + ((j < 4 ? 512 * j : 2048) + 64 * ws) * 16));
-    } else {
-      // ragged last tile: rows past the last key re-read the last key (their scores are
-      // masked to -inf before use)
+    for (int h = 0; h < kHalves; ++h) {
+      const int keyh = key0 + kPartRows * h;
+      const uint32_t ksoff = static_cast<uint32_t>(keyh * a.k_sl) * 2u;
+      // rows past the last key lie past the end of the resource: nothing is read there, and
+      // whatever their scores are, the select that masks them replaces it by -inf
+      if (!kDense || key0 + kKeyTile <= a.Lk) {
 #pragma unroll
-      for (int j = 0; j < 5; ++j) {
-        if (j < nj) {
-          const int rr = min(krow[j], a.Lk - 1 - key0);
-          const uint32_t vo = kvo[j] - static_cast<uint32_t>((krow[j] - rr) * static_cast<int>(a.k_sl)) * 2u;
-          dma16(krs, vo, ksoff, reinterpret_cast<uint16_t*>(st + ((j < 4 ? 512 * j : 2048) + 64 * ws) * 16));
+        for (int j = 0; j < 5; ++j)
+          if (j < nj) dma16(krs, kvo[j], ksoff, dma_dst(st, h, j));
+      } else {
+        // a dense mask is added to the scores, so there they must be finite: rows past the last
+        // key re-read the last key
+#pragma unroll
+        for (int j = 0; j < 5; ++j) {
+          if (j < nj) {
+            const int kr = (64 * (kW * j + ws) + lane) / kRowUnits;
+            const int over = max(0, keyh + kr - (a.Lk - 1));
+            const uint32_t vo = kvo[j] - static_cast<uint32_t>(over * static_cast<int>(a.k_sl)) * 2u;
+            dma16(krs, vo + ksoff, 0u, dma_dst(st, h, j));
+          }
         }
       }
     }
-    // the maxima pass reads K only
-    if (!a.mx_out) {
+  };
+  // DMA of V^T tile t to LDS `st`
+  auto load_v = [&](int gb, int gkvh, int t, uint8_t* st) {
+    const __amdgpu_buffer_rsrc_t vrs = make_rsrc(a.vt + gb * a.v_sb + gkvh * a.v_sh, v_bytes);
+#pragma unroll
+    for (int h = 0; h < kHalves; ++h) {
+      const uint32_t vsoff = static_cast<uint32_t>(t * kKeyTile + kPartRows * h * static_cast<int>(a.v_sd)) * 2u;
 #pragma unroll
       for (int j = 0; j < 5; ++j)
-        if (j < nj) dma16(vrs, vvo[j], vsoff, reinterpret_cast<uint16_t*>(st + kTileBytes + ((j < 4 ? 512 * j : 2048) + 64 * ws) * 16));
+        if (j < nj) dma16(vrs, vvo[j], vsoff, dma_dst(st, h, j));
     }
+  };
+  // eight waves: both tiles into LDS stage `stage` (the maxima pass reads K only)
+  auto load_tile = [&](int gb, int gkvh, int t, int stage) {
+    uint8_t* const st = lds + stage * kStageBytes;
+    load_k(gb, gkvh, t, st);
+    if (!a.mx_out) load_v(gb, gkvh, t, st + kTileBytes);
   };
 
   // LDS operand offsets (bytes).  QK: key row pi(0, n) + 16 kb, piece 2c + half.
@@ -757,7 +796,10 @@ void attn_fwd_kernel(AttnArgs a) {
   for (;;) {
     // first tile of the item, unless the previous item's last tile already fetched it (its
     // stage was last read two steps ago, before the last barrier)
-    if (!issued && g.t_lo < g.t_hi) load_tile(g.b, g.kvh, g.t_lo, step & 1);
+    if (!issued && g.t_lo < g.t_hi) {
+      if constexpr (kW == 8) load_tile(g.b, g.kvh, g.t_lo, step & 1);
+      else load_k(g.b, g.kvh, g.t_lo, lds);
+    }
     issued = false;
     // ---- per-item state: rows, bounds, Q fragment, recurrence state
     const int b = g.b;
@@ -832,7 +874,7 @@ void attn_fwd_kernel(AttnArgs a) {
       // tile t has landed for every wave; every wave is done with the previous step, whose
       // stage the DMA of the next step overwrites
       wait_all_memory();
-      if (pace && w == 0 && (step & (kPaceEvery - 1)) == 1) {
+      if (kW == 8 && pace && w == 0 && (step & (kPaceEvery - 1)) == 1) {
         uint32_t seen = __builtin_amdgcn_readfirstlane(pace_seen);
         for (int spin = 0; spin < kPaceSpins && pace_ahead(step, seen, pace_nw, a.pace_lead); ++spin) {
           __builtin_amdgcn_s_sleep(2);
@@ -849,23 +891,32 @@ void attn_fwd_kernel(AttnArgs a) {
       // chunks 0-1, down to 0 for chunks 6-7) let the wave that is behind win instead, so the
       // two converge and reach the barrier together.
       __builtin_amdgcn_s_setprio(3);
-      if (t + 1 < g.t_hi) {
+      if constexpr (kW == 4) {
+        load_v(b, g.kvh, t, lds + kTileBytes);
+      } else if (t + 1 < g.t_hi) {
         load_tile(b, g.kvh, t + 1, (step + 1) & 1);
       } else if (next_item < n_items && ng.t_lo < ng.t_hi) {
         load_tile(ng.b, ng.kvh, ng.t_lo, (step + 1) & 1);
         issued = true;
       }
-      if (pace && tid == 0 && (step & (kPaceEvery - 1)) == 0)
+      if (kW == 8 && pace && tid == 0 && (step & (kPaceEvery - 1)) == 0)
         pace_seen = __hip_atomic_fetch_add(pace_ctr, kPaceEvery, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + kPaceEvery;
       do {
-        const uint8_t* const st = lds + (step & 1) * kStageBytes;
+        const uint8_t* const st = lds + (kW == 8 ? (step & 1) * kStageBytes : 0);
         const uint8_t* const kp = st + kbyte;
         const uint8_t* const vp = st + vbyte;
 
         const int key0 = t * kKeyTile;
-        if (key0 >= kend_w || key0 + kKeyTile <= kbeg_w) continue;
+        // four waves: both barriers of a tile are every wave's, so a skipped tile only leaves out
+        // the work (S is then defined, not carried over: a value live from an earlier tile
+        // across the barriers would cost registers)
+        const bool skip = key0 >= kend_w || key0 + kKeyTile <= kbeg_w;
+        if (kW == 8 && skip) continue;
         floatx16 s[4];
-        {
+        if (kW == 4 && skip) {
+#pragma unroll
+          for (int kb = 0; kb < 4; ++kb) s[kb] = floatx16{};
+        } else {
           // ---- S^T = K Q^T, c-major (four independent accumulation chains); the K fragments
           // of step c + 1 are read while the MFMAs of step c run
 #pragma unroll
@@ -892,6 +943,8 @@ void attn_fwd_kernel(AttnArgs a) {
         }
         __builtin_amdgcn_sched_barrier(0);
 
+        float mx = -INFINITY, nm = 0.0f;
+        if (kW == 8 || !skip) {
         if (kSoftcap) {
           // sfa:725-727: scores * scale, then softcap * tanh(scores / softcap)
 #pragma unroll
@@ -951,20 +1004,19 @@ void attn_fwd_kernel(AttnArgs a) {
               if (key0 + 64 * half + 16 * kb + i > lim) s[kb][i] = -INFINITY;
         }
         // ---- online softmax in the log2 domain
-        float mx = -INFINITY;
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
           for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[kb][i]);
         const float mx_row = halves_max(mx);
-        if (a.mx_out) {
+        if (kW == 8 && a.mx_out) {
           // maxima pass: the tile's c1-scaled row maximum only
           if (row_live && half == 0) a.mx_out[row * a.mx_stride + t] = mx_row * a.c1;
           continue;
         }
         const float m_new = fmaxf(m_run, mx_row * a.c1);
         const float m_use = m_new == -INFINITY ? 0.0f : m_new;
-        const float nm = -m_use;
+        nm = -m_use;
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
         m_run = m_new;
         if (__ballot(alpha != 1.0f) != 0) {
@@ -977,6 +1029,20 @@ void attn_fwd_kernel(AttnArgs a) {
             dq_run *= alpha;
             dp_run *= alpha;
           }
+        }
+        }
+        if constexpr (kW == 4) {
+          // V^T tile t has landed for every wave and every wave is done with the K tile: the next
+          // K tile (of this item or the next) goes into its place
+          wait_all_memory();
+          __syncthreads();
+          if (t + 1 < g.t_hi) {
+            load_k(b, g.kvh, t + 1, lds);
+          } else if (next_item < n_items && ng.t_lo < ng.t_hi) {
+            load_k(ng.b, ng.kvh, ng.t_lo, lds);
+            issued = true;
+          }
+          if (skip) continue;
         }
         // ---- P, its HiF4 QDQ and the row sum, one 8-key chunk at a time; chunk c of this lane
         // is keys 64 half + 8c .. 8c+7, the B operand of PV k-chunk c.
@@ -1114,7 +1180,8 @@ void attn_fwd_kernel(AttnArgs a) {
     // partially written cache lines.  (kernel-uniform condition: every wave takes the
     // barrier)
     const bool lds_out = !a.o_f32 && !a.mx_out && !a.part_o;
-    uint16_t* const out_rows = reinterpret_cast<uint16_t*>(lds + ((step + 1) & 1) * kStageBytes) + w * (32 * kOutPitch);
+    uint16_t* const out_rows =
+        reinterpret_cast<uint16_t*>(lds + (kW == 8 ? ((step + 1) & 1) * kStageBytes : kTileBytes)) + w * (32 * kOutPitch);
     if (lds_out) __syncthreads();
     if (row_live && !a.mx_out) {
       if (a.part_o) {
