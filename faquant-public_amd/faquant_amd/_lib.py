@@ -238,7 +238,10 @@ def require_device(*tensors: torch.Tensor) -> None:
 
 
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream of ``device`` as a hipStream_t (without building a Stream object, which
+    every launch would pay for: 4 us against 0.3)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 class _ForwardOnly(torch.autograd.Function):

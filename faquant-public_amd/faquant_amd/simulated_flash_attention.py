@@ -185,31 +185,45 @@ def count_tiles(
     pv_group: int,
 ) -> None:
     """The simulator's counters in closed form: its query-tile / key-tile schedule
-    (sfa:623-697, 886-908) replayed without computing anything."""
-    passes = []
+    (sfa:623-697, 886-908) without computing or replaying anything.  All key tiles but the last
+    have one width, and the counters are linear in the number of processed (query tile, key
+    tile) pairs, so each pass needs that number for the full tiles and for the last one.  Only
+    the key tiles that cross the causal diagonal are visited one by one (a decode step has at
+    most one; the loop over every key tile took 1.4 ms of host time at 128k cached keys)."""
     full = query_length // query_chunk
+    tail = full * query_chunk
+    passes = []
     if full:
         passes.append((0, query_chunk, full))
-    tail = full * query_chunk
     if tail < query_length:
         passes.append((tail, query_length - tail, 1))
+    key_tiles = -(-key_length // key_chunk)
+    last_width = key_length - (key_tiles - 1) * key_chunk
     tiles_done = 0
     for q0, rows, tiles in passes:
         if qk_quant:
             _record(stats, "q", head_dim, batch * query_heads * rows * head_dim, qk_group, tiles)
-        for k0 in range(0, key_length, key_chunk):
-            kw = min(k0 + key_chunk, key_length) - k0
-            first = 0
-            if skip_fully_masked and causal:
-                first = max(0, min(tiles, (k0 - (key_length - query_length) - q0) // rows))
-            active = tiles - first
+        if skip_fully_masked and causal:
+            # key tile j is processed by the query tiles from max(0, (j key_chunk - c) // rows) on
+            c = key_length - query_length + q0
+
+            def processed(j):
+                return tiles - max(0, min(tiles, (j * key_chunk - c) // rows))
+
+            n_last = processed(key_tiles - 1)
+            n_all = min(key_tiles - 1, max(0, -(-(rows + c) // key_chunk)))  # tiles every query tile takes
+            n_some = min(key_tiles - 1, max(n_all, -(-(tiles * rows + c) // key_chunk)))  # and any takes
+            n_full = tiles * n_all + sum(processed(j) for j in range(n_all, n_some))
+        else:
+            n_last, n_full = tiles, tiles * (key_tiles - 1)
+        for width, active in ((key_chunk, n_full), (last_width, n_last)):
             if active == 0:
                 continue
             if qk_quant:
-                _record(stats, "k", head_dim, batch * query_heads * kw * head_dim, qk_group, active)
+                _record(stats, "k", head_dim, batch * query_heads * width * head_dim, qk_group, active)
             if pv_quant:
-                _record(stats, "p", kw, batch * query_heads * rows * kw, pv_group, active)
-                _record(stats, "v", head_dim, batch * query_heads * kw * head_dim, pv_group, active)
+                _record(stats, "p", width, batch * query_heads * rows * width, pv_group, active)
+                _record(stats, "v", head_dim, batch * query_heads * width * head_dim, pv_group, active)
             tiles_done += active
     stats["calls"] += 1
     stats["qk_tiles"] += tiles_done
