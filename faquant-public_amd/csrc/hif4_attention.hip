@@ -290,10 +290,11 @@ __device__ __forceinline__ void butterfly32_pair(float& x, float& y) {
 
 // HiF4 QDQ of the fragment: 64-value group g (dims 64 g ..) is chunks 4 g .. 4 g + 3 of lanes
 // n and n + 32; the steps of qdq8 (group maximum of the 4-value maxima, E6M2 scale, micro
-// exponents, elements, a NaN anywhere makes the group NaN).  The sign of qdq8's
-// `w < 0 ? -y : y` is the sign bit of w + 0 (which turns -0 into +0, the one value where
-// the sign bit and w < 0 differ), ORed into y (>= +0); the NaN select runs only when some
-// lane of the wave holds a NaN group.  Both replace per-value v_cndmask, bit for bit.
+// exponents, elements, a NaN anywhere makes the group NaN), with three per-value steps less.
+// The sign of w is copied onto y >= +0: qdq8's `w < 0 ? -y : y` differs only in the sign of a
+// zero that came from w = -0, and a Q value feeds nothing but QK sums that start at +0, which
+// no zero's sign changes.  One unordered comparison tests two values for NaN, and the NaN
+// select runs only when some lane of the wave holds a NaN group.
 template <int LV>
 __device__ __forceinline__ void q_frag_qdq(float (&v)[8][8]) {
   int nan_any = 0;
@@ -308,7 +309,7 @@ __device__ __forceinline__ void q_frag_qdq(float (&v)[8][8]) {
       m3a[cc] = fmaxf(fmaxf(fabsf(w[0]), fabsf(w[1])), fmaxf(fabsf(w[2]), fabsf(w[3])));
       m3b[cc] = fmaxf(fmaxf(fabsf(w[4]), fabsf(w[5])), fmaxf(fabsf(w[6]), fabsf(w[7])));
 #pragma unroll
-      for (int j = 0; j < 8; ++j) nan |= w[j] != w[j];
+      for (int j = 0; j < 8; j += 2) nan |= __builtin_isunordered(w[j], w[j + 1]);
       mx = max(mx, __float_as_int(fmaxf(m3a[cc], m3b[cc])));
     }
     mx = max(mx, lane_swap32(mx));
@@ -326,7 +327,7 @@ __device__ __forceinline__ void q_frag_qdq(float (&v)[8][8]) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const float y = hif4_element(fabsf(w[j]), j < 4 ? qa : qb, j < 4 ? da : db);
-        w[j] = __uint_as_float(__float_as_uint(y) | (__float_as_uint(w[j] + 0.0f) & 0x80000000u));
+        w[j] = __builtin_copysignf(y, w[j]);
       }
     }
     nan_g[g] = nan;
@@ -1230,9 +1231,18 @@ void attn_fwd_kernel(AttnArgs a) {
           for (int r = 0; r < 4; ++r) {
             const float xa = acc[mb][4 * j + r];
             const float q0 = xa * rl;
-            const float x = l > 0.0f ? __builtin_fmaf(__builtin_fmaf(-q0, inv_guard, xa), rl, q0) : 0.0f;
+            const float x = __builtin_fmaf(__builtin_fmaf(-q0, inv_guard, xa), rl, q0);
             val[mb][j][r] = a.o_f32 ? x : bf16_round_hw(x);
           }
+      // rows that saw no key (a select per value only where the wave holds one)
+      if (__ballot(!(l > 0.0f)) != 0) {
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) val[mb][j][r] = l > 0.0f ? val[mb][j][r] : 0.0f;
+      }
       // the o_proj-input QDQ of the output row (qwen3.py:167-171), on the output-dtype values
       if (a.out_levels == 123) qdq_out_row<123>(val, half);
       else if (a.out_levels == 12) qdq_out_row<12>(val, half);

@@ -11,8 +11,8 @@ Reference: src/faquant/wan22_attention.py.  Same public names and signatures:
 accepted and ignored.  P is quantized with the three-level format, as the
 reference kernel's in-register quantizer is.
 
-``make_flash_attention`` fuses rotation, Q/K/V QDQ and attention into two HIP
-launches when ``input_qdq`` comes from ``faquant_qdq`` (it carries its levels);
+``make_flash_attention`` fuses rotation, Q/K/V QDQ and attention into three HIP launches
+(K, V, and the attention, which prepares bf16 Q rows as it loads them) when ``input_qdq`` comes from ``faquant_qdq`` (it carries its levels);
 any other callable is applied as given between the rotation and the kernel.
 
 ``patch_attention_modules(model_module, collector)`` (:231-270) installs the same
@@ -131,11 +131,16 @@ def make_flash_attention(
                 raise NotImplementedError("variable sequence lengths are not supported")
         dim = q.shape[-1]
         scale = float(softmax_scale if softmax_scale is not None else dim**-0.5)
+        q_prep = None
         if fused_prologue:
             # (Smooth-QK) -> rotation (fp32) -> one bf16 cast -> HiF4 QDQ, in one pass per operand
             rot = _ops.HEAD_DIM if qk_rotation else 0
-            qh, _ = _ops.operand_prep(_as_bhld(q), levels=input_qdq.levels, hadamard=rot, smooth=smooth,
-                                      round_dtype=torch.bfloat16)
+            qh = _as_bhld(q)
+            if smooth is None and _ops.raw_q_operand_ok(qh, rot):
+                q_prep = (rot, input_qdq.levels)  # the attention kernel applies it as it loads Q
+            else:
+                qh, _ = _ops.operand_prep(qh, levels=input_qdq.levels, hadamard=rot, smooth=smooth,
+                                          round_dtype=torch.bfloat16)
             kh, _ = _ops.operand_prep(_as_bhld(k), levels=input_qdq.levels, hadamard=rot, smooth=smooth,
                                       smooth_divide=True, round_dtype=torch.bfloat16)
             vt = _ops.operand_prep_vt(_as_bhld(v.to(dtype)), levels=input_qdq.levels)
@@ -149,7 +154,7 @@ def make_flash_attention(
         out = torch.empty((batch, lq, q.shape[2], dim), device=q.device, dtype=torch.bfloat16)
         _ops.attention_fwd(
             qh, kh, vt, lk, causal=False, scale=scale, quant_p=True, p_levels="123",
-            norm_same=quantized_normalizer, out=_as_bhld(out),
+            norm_same=quantized_normalizer, out=_as_bhld(out), q_prep=q_prep,
         )
         return _lib.forward_only(out.type(out_dtype), *inputs)
 
