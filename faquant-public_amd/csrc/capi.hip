@@ -11,6 +11,7 @@
 #include <string>
 
 #include "../../include/faquant_amd.h"
+#include "prep_jobs.h"
 #include "attn_aux.hip"
 #include "attn_decode.h"
 #include "attn_generic.h"
@@ -690,13 +691,102 @@ int faq_operand_prep_vt(const void* x, int in_dtype, int64_t sb, int64_t sh, int
   if ((sb * esz) % 16 || (sh * esz) % 16 || (sl * esz) % 16)
     return fail(FAQ_EINVAL, "faq_operand_prep_vt: strides must keep 16-byte alignment");
   if (static_cast<int64_t>(B) * H * Lpad == 0) return FAQ_OK;
-  faq::OperandPrepVtArgs a{x, sb, sh, sl, B, H, L, Lpad, vt, levels != 0};
+  faq::OperandPrepVtArgs a{x, sb, sh, sl, B, H, L, Lpad, vt, levels != 0, nullptr, 0, 0, 0};
   const dim3 grid(Lpad / 64, B * H);
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (in_dtype == FAQ_F32) launch_prep_vt<float>(a, levels, grid, st);
   else if (in_dtype == FAQ_BF16) launch_prep_vt<__hip_bfloat16>(a, levels, grid, st);
   else launch_prep_vt<__half>(a, levels, grid, st);
   return check_launch("faq_operand_prep_vt");
+}
+
+int faq_operand_prep_jobs(const faq_prep_job* jobs, int n, faq_stream_t stream) {
+  const char* who = "faq_operand_prep_jobs";
+  if (n < 0 || (n > 0 && !jobs)) return fail(FAQ_EINVAL, "%s: bad jobs", who);
+  // one launch for bf16 jobs (at most kPrepJobs row jobs and one V job); any other list runs
+  // its jobs one by one
+  faq::PrepJobsArgs a{};
+  bool one = true;
+  uint64_t blocks = 0;
+  for (int i = 0; i < n; ++i) {
+    const faq_prep_job& p = jobs[i];
+    if (p.in_dtype != FAQ_BF16 || p.round_dtype != FAQ_BF16) one = false;
+    if (static_cast<int64_t>(p.B) * p.H * p.L <= 0) one = false;  // empty or bad: below
+    if (p.vt ? (i != n - 1 || p.codes || p.key_offset || p.smooth || p.hadamard) : a.n == faq::kPrepJobs) one = false;
+    if (!one) break;
+    if (!p.vt) ++a.n;
+  }
+  // the checks of the single entries, through them where the list is run one by one
+  for (int i = 0; i < n; ++i) {
+    const faq_prep_job& p = jobs[i];
+    if (!one) {
+      int rc = FAQ_OK;
+      if (p.vt) {
+        if (p.codes || p.key_offset || p.smooth || p.hadamard)
+          return fail(FAQ_EINVAL, "%s: a transposed job takes no key offset, Smooth-QK, Hadamard or packed rows", who);
+        rc = faq_operand_prep_vt(p.x, p.in_dtype, p.sb, p.sh, p.sl, p.B, p.H, p.L, p.Lpad, p.vt, p.levels, stream);
+      }
+      if (rc == FAQ_OK && p.codes)
+        rc = faq_operand_prep_hif4_kv(p.x, p.in_dtype, p.sb, p.sh, p.sl, p.B, p.H, p.L, p.key_offset, p.off_sh, p.smooth,
+                                      p.smooth_sh, p.smooth_divide, p.hadamard, p.round_dtype, p.levels, p.codes, p.meta,
+                                      p.p_sb, p.p_sh, stream);
+      else if (rc == FAQ_OK && (p.y || !p.vt))
+        rc = faq_operand_prep(p.x, p.in_dtype, p.sb, p.sh, p.sl, p.B, p.H, p.L, p.key_offset, p.off_sh, p.smooth,
+                              p.smooth_sh, p.smooth_divide, p.hadamard, p.round_dtype, nullptr, p.y, p.yb, p.yh, p.yl,
+                              p.levels, stream);
+      if (rc != FAQ_OK) return rc;
+      continue;
+    }
+    if (!p.x || (!p.vt && !p.codes && !p.y) || (p.codes && !p.meta))
+      return fail(FAQ_EINVAL, "%s: null input or output", who);
+    if (p.B < 0 || p.H < 0 || p.L < 0) return fail(FAQ_EINVAL, "%s: negative size", who);
+    if (p.hadamard != 0 && p.hadamard != 64 && p.hadamard != 128)
+      return fail(FAQ_EUNSUP, "%s: Hadamard block must be 64 or 128, got %d", who, p.hadamard);
+    if ((p.levels != 0 || p.codes) && !valid_levels(p.levels))
+      return fail(FAQ_EINVAL, "HiF4 levels must be 123, 12 or 13, got %d", p.levels);
+    if (!aligned16(p.x) || !aligned16(p.y) || !aligned16(p.vt) || !aligned16(p.codes) ||
+        (reinterpret_cast<uintptr_t>(p.meta) & 7u))
+      return fail(FAQ_EINVAL, "%s: pointers must be 16-byte aligned (meta 8)", who);
+    if ((p.sb | p.sh | p.sl) & 7 || (p.y && ((p.yb | p.yh | p.yl) & 7)))
+      return fail(FAQ_EINVAL, "%s: strides must keep 16-byte alignment", who);
+    if (p.codes && (p.p_sb < 0 || p.p_sh < 0)) return fail(FAQ_EINVAL, "%s: negative row strides", who);
+    if (p.B > 65535 || p.H > 65535) return fail(FAQ_EUNSUP, "%s: at most 65535 batches and heads", who);
+    if (p.vt) {
+      if (p.Lpad % 128 || p.Lpad < p.L) return fail(FAQ_EINVAL, "%s: Lpad must be a multiple of 128 >= L", who);
+      a.v = {p.x, p.sb, p.sh, p.sl, p.B, p.H, p.L, p.Lpad, p.vt, p.levels != 0, static_cast<uint16_t*>(p.y),
+             p.yb, p.yh, p.yl};
+      a.v_levels = p.levels;
+      a.v_blocks = p.Lpad / faq::kVtKeys;
+      blocks += static_cast<uint64_t>(a.v_blocks) * p.B * p.H;
+    } else {
+      faq::OperandPrepArgs& d = a.job[i];
+      d.x = p.x;
+      d.sb = p.sb, d.sh = p.sh, d.sl = p.sl;
+      d.B = p.B, d.H = p.H, d.L = p.L;
+      d.key_offset = p.key_offset;
+      d.off_sh = p.off_sh;
+      d.smooth = p.smooth;
+      d.smooth_sh = p.smooth_sh;
+      d.smooth_divide = p.smooth_divide;
+      d.hadamard = p.hadamard;
+      d.div = sqrt_div(p.hadamard);
+      d.y = p.codes ? nullptr : p.y;
+      d.yb = p.yb, d.yh = p.yh, d.yl = p.yl;
+      d.quant = p.levels != 0;
+      d.pk_codes = p.codes;
+      d.pk_meta = p.meta;
+      d.pk_sb = p.p_sb, d.pk_sh = p.p_sh;
+      a.levels[i] = p.levels;
+      a.blocks[i] = (p.L + 16 * faq::kPrepRows - 1) / (16 * faq::kPrepRows);
+      blocks += static_cast<uint64_t>(a.blocks[i]) * p.B * p.H;
+      a.first[i + 1] = static_cast<uint32_t>(blocks);
+    }
+    if (blocks > INT32_MAX) return fail(FAQ_EUNSUP, "%s: too many rows", who);
+  }
+  if (!one || n == 0) return FAQ_OK;
+  hipLaunchKernelGGL(faq::prep_jobs_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), a);
+  return check_launch(who);
 }
 
 int faq_attention_fwd(const uint16_t* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const uint16_t* k, int64_t k_sb,

@@ -929,10 +929,8 @@ __device__ __forceinline__ void pack_hif4_word(const float* y, uint32_t sm_codes
 constexpr int kPrepRows = 2;
 
 template <typename Tin, typename Tround, int LV>
-__global__ __launch_bounds__(256) void operand_prep_kernel(OperandPrepArgs a) {
-  const int h = static_cast<int>(blockIdx.y);
-  const int b = static_cast<int>(blockIdx.z);
-  const int lp0 = static_cast<int>(blockIdx.x) * (16 * kPrepRows) + static_cast<int>(threadIdx.x >> 4);
+__device__ __forceinline__ void operand_prep_block(const OperandPrepArgs& a, int blk, int h, int b) {
+  const int lp0 = blk * (16 * kPrepRows) + static_cast<int>(threadIdx.x >> 4);
   const int part = threadIdx.x & 15;
   const int d0 = part * 8;
   float v[kPrepRows][8];
@@ -999,6 +997,12 @@ __global__ __launch_bounds__(256) void operand_prep_kernel(OperandPrepArgs a) {
   }
 }
 
+template <typename Tin, typename Tround, int LV>
+__global__ __launch_bounds__(256) void operand_prep_kernel(OperandPrepArgs a) {
+  operand_prep_block<Tin, Tround, LV>(a, static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y),
+                                      static_cast<int>(blockIdx.z));
+}
+
 struct OperandPrepVtArgs {
   const void* x;            // V [B, H, L, 128], last stride 1
   int64_t sb, sh, sl;
@@ -1006,19 +1010,21 @@ struct OperandPrepVtArgs {
   int Lpad;                 // multiple of 128, >= L
   uint16_t* vt;             // bf16 [B, H, 128, Lpad]
   int quant;
+  uint16_t* y;              // optional: the same values in natural rows, bf16 [B, H, L, 128] at these strides
+  int64_t yb, yh, yl;
 };
 
 // 64 keys x 128 dims per block: QDQ rows in registers, transpose through LDS, store
 // 16-byte runs of keys for each dim.  Keys >= L are zeros.
+constexpr int kVtKeys = 64;
+constexpr int kVtPitch = kVtKeys + 8;  // uint16 elements per LDS row (16-byte aligned rows)
+
 template <typename Tin, int LV>
-__global__ __launch_bounds__(256) void operand_prep_vt_kernel(OperandPrepVtArgs a) {
-  constexpr int KB = 64;
-  constexpr int PITCH = KB + 8;  // uint16 elements per LDS row (16-byte aligned rows)
-  __shared__ uint16_t tile[128 * PITCH];
-  const int bh = blockIdx.y;
+__device__ __forceinline__ void operand_prep_vt_block(const OperandPrepVtArgs& a, uint16_t* tile, int blk, int bh) {
+  constexpr int KB = kVtKeys, PITCH = kVtPitch;
   const int b = bh / a.H;
   const int h = bh % a.H;
-  const int key0 = blockIdx.x * KB;
+  const int key0 = blk * KB;
   const int part = threadIdx.x & 15;
   const int d0 = part * 8;
   const Tin* x = static_cast<const Tin*>(a.x) + b * a.sb + h * a.sh;
@@ -1036,6 +1042,9 @@ __global__ __launch_bounds__(256) void operand_prep_vt_kernel(OperandPrepVtArgs 
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = Io<Tin>::round(v[i]);
     if (a.quant) qdq8<LV>(v);
+    if (a.y && key < a.L)
+      Io<__hip_bfloat16>::store8(
+          reinterpret_cast<__hip_bfloat16*>(a.y + b * a.yb + h * a.yh + static_cast<int64_t>(key) * a.yl + d0), v);
 #pragma unroll
     for (int i = 0; i < 8; ++i) tile[(d0 + i) * PITCH + rr] = f32_to_bf16_bits_rne(v[i]);
   }
@@ -1049,6 +1058,56 @@ __global__ __launch_bounds__(256) void operand_prep_vt_kernel(OperandPrepVtArgs 
     const uint4 w = *reinterpret_cast<const uint4*>(&tile[d * PITCH + k8]);
     *reinterpret_cast<uint4*>(out + static_cast<int64_t>(d) * a.Lpad + k8) = w;
   }
+}
+
+template <typename Tin, int LV>
+__global__ __launch_bounds__(256) void operand_prep_vt_kernel(OperandPrepVtArgs a) {
+  __shared__ uint16_t tile[128 * kVtPitch];
+  operand_prep_vt_block<Tin, LV>(a, tile, static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y));
+}
+
+// The prologues of one attention call in one launch: up to kPrepJobs row jobs (Q, K, V as bf16
+// rows or packed rows) and one V job that writes V^T and, where wanted, V's natural rows from
+// the same pass.  Block ranges [first[j], first[j + 1]) belong to row job j, the blocks from
+// first[n] on to the V job.  bf16 in and out (the launcher sends other types one by one).
+// What bounds separate launches is their number: each takes 4-12 us for 0.01-20 us of
+// memory traffic, and V^T read back what the V launch had just written.  Same box, launches of
+// three against one, whole calls: 8 x 777 padded prompts 142 -> 128 us, 1999-token prefill
+// 77.7 -> 71.4, a 128k packed decode step 81 -> 71.4.
+constexpr int kPrepJobs = 3;
+
+struct PrepJobsArgs {
+  OperandPrepArgs job[kPrepJobs];
+  int levels[kPrepJobs];
+  int blocks[kPrepJobs];     // position blocks of job j (its grid is blocks x H x B)
+  uint32_t first[kPrepJobs + 1];
+  int n;
+  OperandPrepVtArgs v;
+  int v_levels;
+  int v_blocks;              // key blocks of the V job (Lpad / 64)
+};
+
+__global__ __launch_bounds__(256) void prep_jobs_kernel(PrepJobsArgs a) {
+  typedef __hip_bfloat16 T;
+  __shared__ uint16_t tile[128 * kVtPitch];
+  const uint32_t bx = blockIdx.x;
+  int j = 0;
+  while (j < a.n && bx >= a.first[j + 1]) ++j;
+  const uint32_t i = bx - a.first[j];
+  if (j == a.n) {
+    const int blk = static_cast<int>(i % static_cast<uint32_t>(a.v_blocks)), bh = static_cast<int>(i / static_cast<uint32_t>(a.v_blocks));
+    if (a.v_levels == 12) operand_prep_vt_block<T, 12>(a.v, tile, blk, bh);
+    else if (a.v_levels == 13) operand_prep_vt_block<T, 13>(a.v, tile, blk, bh);
+    else operand_prep_vt_block<T, 123>(a.v, tile, blk, bh);
+    return;
+  }
+  const OperandPrepArgs& p = a.job[j];
+  const uint32_t nb = static_cast<uint32_t>(a.blocks[j]), hb = i / nb;
+  const int blk = static_cast<int>(i % nb), h = static_cast<int>(hb % static_cast<uint32_t>(p.H)),
+            b = static_cast<int>(hb / static_cast<uint32_t>(p.H));
+  if (a.levels[j] == 12) operand_prep_block<T, T, 12>(p, blk, h, b);
+  else if (a.levels[j] == 13) operand_prep_block<T, T, 13>(p, blk, h, b);
+  else operand_prep_block<T, T, 123>(p, blk, h, b);
 }
 
 }  // namespace faq

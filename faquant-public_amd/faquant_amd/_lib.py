@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 
 import torch
 
@@ -84,6 +85,12 @@ class ActOpts(ctypes.Structure):
 
 
 _act_opts_p = ctypes.POINTER(ActOpts)
+
+
+# faq_prep_job (csrc/prep_jobs.h), packed with the C layout: x, in_dtype, sb, sh, sl, B, H, L,
+# key_offset, off_sh, smooth, smooth_sh, smooth_divide, hadamard, round_dtype, y, yb, yh, yl, levels,
+# codes, meta, p_sb, p_sh, vt, Lpad (one pack call: a ctypes structure takes 5 us to fill)
+PREP_JOB = struct.Struct("@PiqqqiiiPqPqiiiPqqqiPPqqPi0q")
 
 _SIGNATURES = {
     "faq_last_error": ([], ctypes.c_char_p),
@@ -188,6 +195,8 @@ _SIGNATURES = {
 }
 
 EXPORTED = tuple(_SIGNATURES)
+# calls of this package only (csrc/prep_jobs.h), outside the public C ABI
+_INTERNAL = {"faq_operand_prep_jobs": ([_vp, _c_int, _vp], _c_int)}
 
 _lib = None
 
@@ -202,7 +211,7 @@ def load() -> ctypes.CDLL:
                 "(python faquant-public_amd/build.py, or __graft_entry__.build())"
             )
         lib = ctypes.CDLL(LIB_PATH)
-        for name, (args, res) in _SIGNATURES.items():
+        for name, (args, res) in {**_SIGNATURES, **_INTERNAL}.items():
             fn = getattr(lib, name)
             fn.argtypes = args
             fn.restype = res

@@ -278,9 +278,10 @@ def pquant_groups(p: torch.Tensor, levels: str) -> torch.Tensor:
 
 
 def _bhld_strides(x: torch.Tensor) -> tuple[int, int, int]:
-    if x.stride(-1) != 1:
+    sb, sh, sl, sd = x.stride()
+    if sd != 1:
         raise ValueError("operands need a unit stride along head_dim")
-    return x.stride(0), x.stride(1), x.stride(2)
+    return sb, sh, sl
 
 
 def operand_prep(
@@ -513,6 +514,51 @@ def operand_prep_vt(v: torch.Tensor, *, levels: str | None) -> torch.Tensor:
         )
     )
     return vt
+
+
+def prep_job(x: torch.Tensor, *, levels: str | None, out: torch.Tensor | None = None,
+             packed: PackedHiF4KV | None = None, start: int = 0, vt: torch.Tensor | None = None, hadamard: int = 0,
+             key_offset: torch.Tensor | None = None, smooth: torch.Tensor | None = None, smooth_divide: bool = False,
+             round_dtype: torch.dtype | None = None):
+    """One operand for ``operand_prep_jobs``: ``operand_prep`` into the bf16 view ``out``,
+    ``pack_operand`` into rows ``start`` .. of ``packed`` (the caller sets its length), or ``operand_prep_vt`` into ``vt``
+    (and natural rows into ``out`` where given)."""
+    _lib.require_device(x, out, vt, key_offset, smooth)
+    if x.ndim != 4 or x.shape[-1] != HEAD_DIM:
+        raise NotImplementedError("the HIP operand prologue supports [B, H, L, 128] tensors")
+    B, H, L, _ = x.shape
+    sb, sh, sl = _bhld_strides(x)
+    off, off_sh = _per_head(key_offset, H, x.device)
+    sm, sm_sh = _per_head(smooth, H, x.device)
+    y = codes = meta = yb = yh = yl = p_sb = p_sh = vt_ptr = lpad = 0
+    if packed is not None:
+        if tuple(packed.codes.shape[:2]) != (B, H) or start < 0 or start + L > packed.capacity:
+            raise ValueError(f"rows {start}..{start + L} of a packed cache of shape {tuple(packed.codes.shape[:3])}")
+        if not levels:
+            raise ValueError("the packed HiF4 form needs HiF4 levels")
+        d = packed.descriptor()
+        codes, meta, p_sb, p_sh = d.codes + start * 64, d.meta + start * 8, d.sb, d.sh
+    elif out is not None:
+        _checked_out(out, x, (B, H, L, HEAD_DIM), torch.bfloat16, unit_last_only=True)
+        y = out.data_ptr()
+        yb, yh, yl, _ = out.stride()
+    if vt is not None:
+        if tuple(vt.shape) != (B, H, HEAD_DIM, _pad_keys(L)) or vt.dtype != torch.bfloat16 or not vt.is_contiguous():
+            raise ValueError(f"vt must be a contiguous bf16 tensor of shape {(B, H, HEAD_DIM, _pad_keys(L))}")
+        vt_ptr, lpad = vt.data_ptr(), vt.shape[-1]
+    code = _lib.dtype_code(x.dtype)
+    job = _lib.PREP_JOB.pack(
+        x.data_ptr(), code, sb, sh, sl, B, H, L, _lib.ptr(off) or 0, off_sh, _lib.ptr(sm) or 0, sm_sh, bool(smooth_divide),
+        int(hadamard or 0), code if round_dtype is None else _lib.dtype_code(round_dtype), y, yb, yh, yl,
+        int(levels) if levels else 0, codes, meta, p_sb, p_sh, vt_ptr, lpad)
+    # the tensors stay referenced until the launch
+    return job, (x, out, packed, vt, off, sm)
+
+
+def operand_prep_jobs(jobs: list, device: torch.device) -> None:
+    """The operand prologues of one attention call (``prep_job`` each, a ``vt`` job last): one
+    launch for bf16 operands, the outputs of the single entries bit for bit."""
+    _lib.check(_lib.load().faq_operand_prep_jobs(b"".join(j for j, _ in jobs), len(jobs), _lib.stream_ptr(device)))
 
 
 @dataclass

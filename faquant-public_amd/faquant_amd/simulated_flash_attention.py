@@ -274,67 +274,79 @@ def _append_allowed(module, name: str, state, tensor: torch.Tensor, query_length
     )
 
 
-def _key_operand(module, key: torch.Tensor, *, enabled: bool, query_length: int, levels: str, **prep) -> torch.Tensor:
-    """bf16 K operand [B, Hkv, Lk, 128]; with K quantization it doubles as the decode QDQ
-    cache ``faquant_k_matmul_qdq_cache`` (sfa:243-289): a decode step quantizes only the
-    appended position into a capacity-padded buffer.  K QDQ (and the optional Q/K
-    prologue ``prep`` of operand_prep) is token-local, so this is bitwise equal to
-    quantizing the whole cache again."""
-    name = "faquant_k_matmul_qdq_cache"
-    states = getattr(module, _KV_STATE, None) or {}
-    if not enabled:
-        setattr(module, name, None)
-        states.pop("k", None)
-        setattr(module, _KV_STATE, states)
-        return _ops.operand_prep(key, levels=None, **prep)[0]
-    B, H, L, D = key.shape
-    st = states.get("k")
-    if _append_allowed(module, name, st, key, query_length):
-        buf = st["buf"]
+def _qdq_cache(module, which: str, tensor: torch.Tensor, query_length: int):
+    """The decode QDQ cache ``faquant_{k,v}_matmul_qdq_cache`` of ``tensor`` (sfa:243-289), a
+    capacity-padded natural [B, Hkv, cap, 128] buffer: its [B, Hkv, L, 128] view, the first
+    position that this call still has to quantize into it (0, or L - 1 of a decode step that
+    appends: the QDQ is token-local, so that is bitwise a full re-quantization), and the function
+    that attaches it to the module once the launch that fills it is enqueued."""
+    name = f"faquant_{which}_matmul_qdq_cache"
+    states = getattr(module, _KV_STATE, None)
+    if states is None:
+        states = {}
+        setattr(module, _KV_STATE, states)  # one dict for K and V
+    B, H, L, D = tensor.shape
+    st = states.get(which)
+    start = 0
+    if _append_allowed(module, name, st, tensor, query_length):
+        buf, start = st["buf"], L - 1
         if L > buf.shape[2]:
-            grown = torch.empty((B, H, _cache_capacity(L + _KV_GROWTH), D), device=key.device, dtype=torch.bfloat16)
+            grown = torch.empty((B, H, _cache_capacity(L + _KV_GROWTH), D), device=tensor.device, dtype=torch.bfloat16)
             grown[:, :, : L - 1].copy_(buf[:, :, : L - 1])
             buf = grown
-        _ops.operand_prep(key[:, :, L - 1 :], levels=levels, out=buf[:, :, L - 1 : L], **prep)
     else:
-        buf = torch.empty((B, H, _cache_capacity(L), D), device=key.device, dtype=torch.bfloat16)
-        _ops.operand_prep(key, levels=levels, out=buf[:, :, :L], **prep)
+        buf = torch.empty((B, H, _cache_capacity(L), D), device=tensor.device, dtype=torch.bfloat16)
     view = buf[:, :, :L]
-    states["k"] = dict(buf=buf, view=view, length=L, device=key.device, dtype=key.dtype, lead=(B, H))
-    setattr(module, _KV_STATE, states)
-    setattr(module, name, view)
-    return view
 
-
-def _value_operand(module, value: torch.Tensor, *, enabled: bool, query_length: int, levels: str) -> torch.Tensor:
-    """bf16 V operand [B, Hkv, Lk, 128] in natural rows; with V quantization it doubles as
-    the decode QDQ cache ``faquant_v_matmul_qdq_cache`` (sfa:243-289), a capacity-padded
-    buffer where a decode step quantizes only the appended position.  The prefill kernels
-    take a transposed copy (transposed_values)."""
-    name = "faquant_v_matmul_qdq_cache"
-    states = getattr(module, _KV_STATE, None) or {}
-    if not enabled:
-        setattr(module, name, None)
-        states.pop("v", None)
+    def attach():
+        states[which] = dict(buf=buf, view=view, length=L, device=tensor.device, dtype=tensor.dtype, lead=(B, H))
         setattr(module, _KV_STATE, states)
-        return value
-    B, H, L, D = value.shape
-    st = states.get("v")
-    if _append_allowed(module, name, st, value, query_length):
-        buf = st["buf"]
-        if L > buf.shape[2]:
-            grown = torch.empty((B, H, _cache_capacity(L + _KV_GROWTH), D), device=value.device, dtype=torch.bfloat16)
-            grown[:, :, : L - 1].copy_(buf[:, :, : L - 1])
-            buf = grown
-        _ops.operand_prep(value[:, :, L - 1 :], levels=levels, out=buf[:, :, L - 1 : L])
-    else:
-        buf = torch.empty((B, H, _cache_capacity(L), D), device=value.device, dtype=torch.bfloat16)
-        _ops.operand_prep(value, levels=levels, out=buf[:, :, :L])
-    view = buf[:, :, :L]
-    states["v"] = dict(buf=buf, view=view, length=L, device=value.device, dtype=value.dtype, lead=(B, H))
+        setattr(module, name, view)
+
+    return view, start, attach
+
+
+def _no_cache(module, which: str) -> None:
+    setattr(module, f"faquant_{which}_matmul_qdq_cache", None)
+    states = getattr(module, _KV_STATE, None) or {}
+    states.pop(which, None)
     setattr(module, _KV_STATE, states)
-    setattr(module, name, view)
-    return view
+
+
+def _kv_operands(module, key: torch.Tensor, value: torch.Tensor, *, query_length: int, qk_quant: bool, pv_quant: bool,
+                 levels, k_prep: dict, transposed: bool, q_job=None):
+    """bf16 K and V operands through the module's decode caches: K [B, Hkv, Lk, 128] with its
+    prologue ``k_prep``, and V in natural rows or, with ``transposed``, as V^T.  Their prologues
+    and ``q_job`` run as one launch for bf16 tensors."""
+    attach = []
+    if qk_quant:
+        k_op, k0, done = _qdq_cache(module, "k", key, query_length)
+        attach.append(done)
+    else:
+        _no_cache(module, "k")
+        k_op, k0 = torch.empty(key.shape, device=key.device, dtype=torch.bfloat16), 0
+    jobs = [] if q_job is None else [q_job]
+    jobs.append(_ops.prep_job(key[:, :, k0:], levels=levels["k"] if qk_quant else None, out=k_op[:, :, k0:], **k_prep))
+    v_op, v0 = value, 0
+    if pv_quant:
+        v_op, v0, done = _qdq_cache(module, "v", value, query_length)
+        attach.append(done)
+    else:
+        _no_cache(module, "v")
+    v_levels = levels["v"] if pv_quant else None
+    vt = None
+    if transposed and v0 == 0:
+        B, H, L, D = value.shape
+        vt = torch.empty((B, H, D, _ops._pad_keys(L)), device=value.device, dtype=torch.bfloat16)
+        jobs.append(_ops.prep_job(value, levels=v_levels, out=v_op if pv_quant else None, vt=vt))
+    elif pv_quant:
+        jobs.append(_ops.prep_job(value[:, :, v0:], levels=v_levels, out=v_op[:, :, v0:]))
+    _ops.operand_prep_jobs(jobs, key.device)
+    for done in attach:
+        done()
+    if not transposed:
+        return k_op, v_op
+    return k_op, transposed_values(v_op) if vt is None else vt
 
 
 def transposed_values(v: torch.Tensor) -> torch.Tensor:
@@ -349,32 +361,38 @@ def _packed_cache_enabled(module, qk_quant: bool, pv_quant: bool) -> bool:
     return bool(getattr(module, "faquant_kv_cache_packed", False)) and qk_quant and pv_quant
 
 
-def _packed_operands(module, key: torch.Tensor, value: torch.Tensor, *, query_length: int, levels, prep: dict):
+def _packed_operands(module, key: torch.Tensor, value: torch.Tensor, *, query_length: int, levels, prep: dict,
+                     q_job=None):
     """The decode K/V caches of sfa:243-289 held packed (4.5 bits per value, PackedHiF4KV):
     ``faquant_k_matmul_qdq_cache`` / ``faquant_v_matmul_qdq_cache`` are PackedHiF4KV objects
     whose rows decode to the bf16 QDQ values of the unpacked caches.  A decode step packs
     only the appended position (the same append condition); anything else packs the whole
-    tensor.  K takes the operand prologue ``prep`` (Hadamard, Smooth-QK, key offset)."""
+    tensor.  K takes the operand prologue ``prep`` (Hadamard, Smooth-QK, key offset).  The
+    prologues and ``q_job`` run as one launch for bf16 tensors."""
     states = getattr(module, _KV_STATE, None) or {}
     states.pop("k", None)  # no bf16 caches beside the packed ones
     states.pop("v", None)
     caches = []
+    jobs = [] if q_job is None else [q_job]
     for name, t, lv, pre in (("k", key, levels["k"], prep), ("v", value, levels["v"], {})):
         attr = f"faquant_{name}_matmul_qdq_cache"
         st = states.get("packed_" + name)
         B, H, L, _ = t.shape
+        start = 0
         if _append_allowed(module, attr, st, t, query_length):
-            cache = st["buf"]
+            cache, start = st["buf"], L - 1
             if L > cache.capacity:
                 cache = cache.grow(_cache_capacity(L + _KV_GROWTH))
-            _ops.pack_operand(t[:, :, L - 1 :], levels=lv, out=cache, start=L - 1, **pre)
         else:
             cache = _ops.PackedHiF4KV(B, H, _cache_capacity(L), t.device, lv)
-            _ops.pack_operand(t, levels=lv, out=cache, **pre)
-        cache.length = L
-        states["packed_" + name] = dict(buf=cache, view=cache, length=L, device=t.device, dtype=t.dtype, lead=(B, H))
-        setattr(module, attr, cache)
+        jobs.append(_ops.prep_job(t[:, :, start:], levels=lv, packed=cache, start=start, **pre))
         caches.append(cache)
+    _ops.operand_prep_jobs(jobs, key.device)
+    for name, t, cache in (("k", key, caches[0]), ("v", value, caches[1])):
+        cache.length = t.shape[2]
+        states["packed_" + name] = dict(buf=cache, view=cache, length=t.shape[2], device=t.device, dtype=t.dtype,
+                                        lead=tuple(t.shape[:2]))
+        setattr(module, f"faquant_{name}_matmul_qdq_cache", cache)
     setattr(module, _KV_STATE, states)
     return caches
 
@@ -391,11 +409,6 @@ def kv_operands_and_attend(module, q_op: torch.Tensor, key: torch.Tensor, value:
     if q_prep is not None:
         attn = dict(attn, q_prep=q_prep)
 
-    def prepared_q():
-        if q_prep is None:
-            return q_op
-        return _ops.operand_prep(q_op, levels=q_prep[1], hadamard=q_prep[0], round_dtype=torch.bfloat16)[0]
-
     key_length = key.shape[2]
     B, Hq, Hkv = q_op.shape[0], q_op.shape[1], key.shape[1]
     plain = not (attn.get("ranges") is not None or attn.get("softcap") or attn.get("pv_probe") is not None
@@ -406,18 +419,23 @@ def kv_operands_and_attend(module, q_op: torch.Tensor, key: torch.Tensor, value:
               and _ops._split_count(B, Hq, Hkv, query_length, key_length, _ops._device_cus(q_op.device)) > 1)
     dkw = dict(causal=attn["causal"], scale=attn["scale"], quant_p=attn["quant_p"], p_levels=attn["p_levels"],
                norm_same=attn["norm_same"], out=attn["out"], row_den=attn.get("row_den"))
+    # the decode kernel takes prepared queries: their prologue joins K's and V's
+    q_job = None
+    if decode and q_prep is not None:
+        raw, q_op = q_op, torch.empty(q_op.shape, device=q_op.device, dtype=torch.bfloat16)
+        q_job = _ops.prep_job(raw, levels=q_prep[1], hadamard=q_prep[0], round_dtype=torch.bfloat16, out=q_op)
     if _packed_cache_enabled(module, qk_quant, pv_quant):
-        kp, vp = _packed_operands(module, key, value, query_length=query_length, levels=levels, prep=k_prep)
+        kp, vp = _packed_operands(module, key, value, query_length=query_length, levels=levels, prep=k_prep, q_job=q_job)
         if decode:
-            return _ops.attention_decode(prepared_q(), key_length, packed=(kp, vp), **dkw)
+            return _ops.attention_decode(q_op, key_length, packed=(kp, vp), **dkw)
         k_op, _ = _ops.operand_prep(key, levels=levels["k"], **k_prep)
         vt = _ops.operand_prep_vt(value, levels=levels["v"])
         return _ops.attention_fwd(q_op, k_op, vt, key_length, **attn)
-    k_op = _key_operand(module, key, enabled=qk_quant, query_length=query_length, levels=levels["k"], **k_prep)
-    v_op = _value_operand(module, value, enabled=pv_quant, query_length=query_length, levels=levels["v"])
+    k_op, v_op = _kv_operands(module, key, value, query_length=query_length, qk_quant=qk_quant, pv_quant=pv_quant,
+                              levels=levels, k_prep=k_prep, transposed=not decode, q_job=q_job)
     if decode:
-        return _ops.attention_decode(prepared_q(), key_length, k=k_op, v=v_op, **dkw)
-    return _ops.attention_fwd(q_op, k_op, transposed_values(v_op), key_length, **attn)
+        return _ops.attention_decode(q_op, key_length, k=k_op, v=v_op, **dkw)
+    return _ops.attention_fwd(q_op, k_op, v_op, key_length, **attn)
 
 
 def _unit_last(t: torch.Tensor) -> torch.Tensor:
