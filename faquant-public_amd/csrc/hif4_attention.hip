@@ -406,46 +406,6 @@ __device__ __forceinline__ float p_arg(float s, float c1, float nm) {
   return kExact ? (s * c1) + nm : __builtin_fmaf(s, c1, nm);
 }
 
-__device__ __forceinline__ float floor2(float x) { return __uint_as_float(__float_as_uint(x) & 0xFF800000u); }
-
-// max of two non-negative floats as an integer max of their bit patterns
-__device__ __forceinline__ float fmax_nonneg(float a, float b) {
-  return __uint_as_float(max(__float_as_uint(a), __float_as_uint(b)));
-}
-
-// Per-lane constants of the HiF4 QDQ of one 64-key P group (p >= 0) with maximum m1.
-struct PQuant {
-  float rec4;  // 4 rec
-  float s16;   // s / 16
-};
-
-// Same values as hif4_scale (hif4.py:91-115) for m1 >= 0: s0 = bf16(m1 bf16(1/div)),
-// clamped to [2^-48, 49152] (integer clamp of the non-negative bit pattern), E6M2
-// round-half-even on the bits, and rec = bf16(1/s): 1/s = 2^-e / (1 + m/4) lies far from
-// every bf16 rounding boundary, so the 1-ulp hardware reciprocal rounds to the same bf16.
-template <int LV>
-__device__ __forceinline__ PQuant pquant_setup(float m1) {
-  const float s0 = bf16_round_hw(m1 * divisor_reciprocal<LV>());
-  uint32_t b = min(max(__float_as_uint(s0), 0x27800000u), 0x47400000u);
-  b = (b + 0x000FFFFFu + ((b >> 21) & 1u)) & 0xFFE00000u;
-  const float sc = __uint_as_float(b);
-  const float rec = bf16_round_hw(__builtin_amdgcn_rcpf(sc));
-  PQuant q;
-  q.rec4 = rec * 4.0f;
-  q.s16 = sc * 0.0625f;
-  return q;
-}
-
-// 4K for the micro exponent k of one 4-key group (K = 2^k), from x = floor2 of its
-// v-maximum 4 t3 and e = 4 2^e2 of its 8-key group (levels 123).  Both are 0 or powers of
-// two; med3 clamps floor2(4 t3) into [4 2^e2, 16], which is the reference's lv2 + lv3 rule
-// (hif4.py:200-213): t3 < 2 gives K = 2^e2, t3 in [2, 4) gives K = 2, t3 >= 4 gives K = 4.
-__device__ __forceinline__ float k4_of(float x, float e) { return __builtin_amdgcn_fmed3f(x, e, 16.0f); }
-
-// 1/K of 4K (both exact powers of two): an integer subtraction of the exponent fields,
-// 2^-k = (127 - k) << 23 = (256 << 23) - ((129 + k) << 23).
-__device__ __forceinline__ float inv_k_of(float k4) { return __uint_as_float(0x80000000u - __float_as_uint(k4)); }
-
 // HiF4 QDQ in place of one 8-key group g[0..7] (two 4-key groups) of a lane's P group,
 // with the reference's roundings (hif4.py:255-271):
 //   v = RN(p 4 rec), exactly 4 RN(p rec) (the exact scaling by 4 commutes with rounding);

@@ -175,6 +175,49 @@ __device__ __forceinline__ float group_max8(float v) {
   return __int_as_float(u);
 }
 
+// NaN-propagating maximum of three magnitudes (one v_maximum3_f32).
+__device__ __forceinline__ float abs_max3_nan(float a, float b, float c) {
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(a), fabsf(b)), fabsf(c));
+}
+
+// qdq8 without metadata outputs, the same values in fewer instructions (all callers of this
+// form are bound by VALU issue): the maxima propagate NaN, so the group maximum itself says
+// whether the group holds one (a positive NaN's bits are above every number's in the integer
+// maximum across lanes); the micro exponents come from exponent masks and med3 (k4_of)
+// instead of compares and selects; the sign of w + 0 (which turns -0 into +0, the one value
+// where the sign bit and w < 0 differ) is copied onto y; the NaN select runs only where some
+// lane of the wave needs it.
+template <int LV>
+__device__ __forceinline__ void qdq8_values(float* v) {
+  const float m3a = __builtin_elementwise_maximum(abs_max3_nan(v[0], v[1], v[2]), fabsf(v[3]));
+  const float m3b = __builtin_elementwise_maximum(abs_max3_nan(v[4], v[5], v[6]), fabsf(v[7]));
+  const float m1 = group_max8(__builtin_elementwise_maximum(m3a, m3b));
+  const PQuant q = pquant_setup<LV>(m1);
+  // floor2 of 4 t3, t3 = RN(m3 rec)
+  const float xa = floor2(m3a * q.rec4), xb = floor2(m3b * q.rec4);
+  float k4a, k4b;
+  if (LV == 123) {
+    const float e2 = __builtin_amdgcn_fmed3f(fmaxf(xa, xb) * 0.5f, 4.0f, 8.0f);
+    k4a = k4_of(xa, e2);
+    k4b = k4_of(xb, e2);
+  } else if (LV == 12) {
+    k4a = k4b = __builtin_amdgcn_fmed3f(fmaxf(xa, xb), 4.0f, 8.0f);
+  } else {
+    k4a = __builtin_amdgcn_fmed3f(xa, 4.0f, 8.0f);
+    k4b = __builtin_amdgcn_fmed3f(xb, 4.0f, 8.0f);
+  }
+  const float qa = q.rec4 * inv_k_of(k4a), qb = q.rec4 * inv_k_of(k4b);  // 4 rec 2^-k
+  const float da = k4a * q.s16, db = k4b * q.s16;                          // s 2^k / 4
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    v[i] = __builtin_copysignf(hif4_element(fabsf(v[i]), i < 4 ? qa : qb, i < 4 ? da : db), v[i] + 0.0f);
+  const bool nan = m1 != m1;
+  if (__ballot(nan) != 0) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = nan ? __builtin_nanf("") : v[i];
+  }
+}
+
 // HiF4 QDQ of the 8 values a lane owns (signed, |x| based).  Lanes 8j..8j+7 must hold
 // one 64-value group in order.  `nan_in_group` reproduces the reference's NaN
 // propagation: a NaN anywhere in a block makes the whole block NaN.
@@ -504,7 +547,7 @@ __global__ __launch_bounds__(256) void act_qdq_rows_kernel(ActQdqArgs a) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = Io<T>::round(v[i]);
   }
-  if (a.quant) qdq8<LV>(v);
+  if (a.quant) qdq8_values<LV>(v);
   if (have) Io<T>::store8(y + c0, v);
 }
 
@@ -547,13 +590,14 @@ struct ActRowArgs {
 // coalesced load / store layout and the QDQ layout: 8 consecutive lanes hold one 64-value
 // group).  LDS holds one fp32 copy of the row for the permutation gather and for the
 // butterfly stages that cross lanes.
-// Value j sits at lds_pad(j) = j + j / 8: one spare word after every 8 values, so lanes that
-// write or read their 8-value chunks (8 words apart), and the first butterfly pass over LDS
-// (stride 8), touch distinct banks.
+// Value j sits at lds_pad(j) = j + 4 (j / 32): four spare words after every 32 values, so that a
+// chunk is two aligned 16-byte accesses and the half-wave of a butterfly read (stride 8: four
+// runs of 8 words, 144 words apart; larger strides: 32 consecutive words) touches distinct
+// banks.  The gather's copy of the row is unpadded (its reads are random anyway).
 __host__ __device__ constexpr size_t act_row_lds_bytes(int cols) {
   return static_cast<size_t>(cols + cols / 8) * sizeof(float);
 }
-__device__ __forceinline__ int lds_pad(int j) { return j + (j >> 3); }
+__host__ __device__ constexpr int lds_pad(int j) { return j + ((j >> 5) << 2); }
 
 // First value of chunk r of lane `tid`.
 template <int R, int NT>
@@ -582,18 +626,19 @@ __device__ __forceinline__ void fwht_in_chunks(float (&v)[R][8]) {
 // two passes instead of three with radix 8; 12-18% less time at 4096 and 12288 features).
 constexpr int kActRadix = 4;
 
-// One pass over the LDS row of the LR stages of stride s, 2 s, .. (LR = 1 .. 4; s a
-// multiple of 8, 2^LR s dividing the block): group g holds the 2^LR values j0 + m s.
-template <int LR, int NT, typename RT = float>
-__device__ __forceinline__ void fwht_lds_pass(float* lds, int cols, int ls, int tid) {
+// One pass over the LDS row of the LR stages of stride s = 2^LS, 2 s, .. (LR = 1 .. 4; LS = 3, 7
+// or 11; 2^LR s dividing the block): group g holds the 2^LR values j0 + m s.  j0 has
+// no carry into m s (their bits are disjoint), so value m sits at lds_pad(j0) +
+// lds_pad(m s), a constant offset.
+template <int LR, int LS, int NT, typename RT = float>
+__device__ __forceinline__ void fwht_lds_pass(float* lds, int cols, int tid) {
   constexpr int kRad = 1 << LR;
-  const int s = 1 << ls;
-  const int as = s + (s >> 3);  // j0 + m s sits at lds_pad(j0) + m (s + s / 8)
+  constexpr int s = 1 << LS;
   for (int g = tid; g < (cols >> LR); g += NT) {
-    const int a0 = lds_pad(((g >> ls) << (ls + LR)) | (g & (s - 1)));
+    float* const p = lds + lds_pad(((g >> LS) << (LS + LR)) | (g & (s - 1)));
     float w[kRad];
 #pragma unroll
-    for (int m = 0; m < kRad; ++m) w[m] = lds[a0 + m * as];
+    for (int m = 0; m < kRad; ++m) w[m] = p[lds_pad(m * s)];
 #pragma unroll
     for (int t = 1; t < kRad; t <<= 1)
 #pragma unroll
@@ -604,8 +649,16 @@ __device__ __forceinline__ void fwht_lds_pass(float* lds, int cols, int ls, int 
           w[m + t] = Io<RT>::round(l - h);
         }
 #pragma unroll
-    for (int m = 0; m < kRad; ++m) lds[a0 + m * as] = w[m];
+    for (int m = 0; m < kRad; ++m) p[lds_pad(m * s)] = w[m];
   }
+}
+
+template <int LS, int NT, typename RT>
+__device__ __forceinline__ void fwht_lds_stages(float* lds, int cols, int lr, int tid) {
+  if (lr >= 4) fwht_lds_pass<4, LS, NT, RT>(lds, cols, tid);
+  else if (lr == 3) fwht_lds_pass<3, LS, NT, RT>(lds, cols, tid);
+  else if (lr == 2) fwht_lds_pass<2, LS, NT, RT>(lds, cols, tid);
+  else fwht_lds_pass<1, LS, NT, RT>(lds, cols, tid);
 }
 
 template <int R, int NT>
@@ -613,9 +666,7 @@ __device__ __forceinline__ void row_to_lds(const float (&v)[R][8], float* lds, i
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int c0 = act_c0<R, NT>(tid, r);
-    if (c0 < cols)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) lds[lds_pad(c0) + i] = v[r][i];
+    if (c0 < cols) Io<float>::store8(lds + lds_pad(c0), v[r]);
   }
 }
 
@@ -624,9 +675,7 @@ __device__ __forceinline__ void row_from_lds(float (&v)[R][8], const float* lds,
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int c0 = act_c0<R, NT>(tid, r);
-    if (c0 < cols)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[r][i] = lds[lds_pad(c0) + i];
+    if (c0 < cols) Io<float>::load8(lds + lds_pad(c0), v[r]);
   }
 }
 
@@ -644,13 +693,15 @@ __device__ __forceinline__ void fwht_row_raw(float (&v)[R][8], float* lds, int c
   if (b > 8) {
     row_to_lds<R, NT>(v, lds, cols, tid);
     const int lb = __builtin_ctz(b);
-    for (int ls = 3; ls < lb; ls += kActRadix) {
+    __syncthreads();
+    fwht_lds_stages<3, NT, RT>(lds, cols, lb - 3, tid);
+    if (lb > 3 + kActRadix) {
       __syncthreads();
-      const int lr = min(kActRadix, lb - ls);
-      if (lr == 4) fwht_lds_pass<4, NT, RT>(lds, cols, ls, tid);
-      else if (lr == 3) fwht_lds_pass<3, NT, RT>(lds, cols, ls, tid);
-      else if (lr == 2) fwht_lds_pass<2, NT, RT>(lds, cols, ls, tid);
-      else fwht_lds_pass<1, NT, RT>(lds, cols, ls, tid);
+      fwht_lds_stages<3 + kActRadix, NT, RT>(lds, cols, lb - 3 - kActRadix, tid);
+    }
+    if (lb > 3 + 2 * kActRadix) {
+      __syncthreads();
+      fwht_lds_stages<3 + 2 * kActRadix, NT, RT>(lds, cols, lb - 3 - 2 * kActRadix, tid);
     }
     __syncthreads();
     row_from_lds<R, NT>(v, lds, cols, tid);
@@ -702,11 +753,29 @@ __device__ __forceinline__ void generalized_row(float (&v)[R][8], float* lds, in
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int c0 = act_c0<R, NT>(tid, r);
-    if (c0 < cols)
+    if (c0 < cols) {
+      Io<float>::load8(lds + lds_pad(c0), v[r]);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[r][i] = lds[lds_pad(c0) + i] / d;
+      for (int i = 0; i < 8; ++i) v[r][i] = v[r][i] / d;
+    }
   }
   __syncthreads();
+}
+
+// Eight values rounded to T (bf16: two per conversion instruction).
+template <typename T>
+__device__ __forceinline__ void round8(float* v) {
+  if constexpr (std::is_same<T, __hip_bfloat16>::value) {
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+      const uint32_t u = pack2_bf16_hw(v[i], v[i + 1]);
+      v[i] = __uint_as_float(u << 16);
+      v[i + 1] = __uint_as_float(u & 0xFFFF0000u);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = Io<T>::round(v[i]);
+  }
 }
 
 // v as a T value before the companding quotient.  v is the QDQ output (a HiF4 value: at most
@@ -738,6 +807,13 @@ __global__ __launch_bounds__(256) void compand_rcp_kernel(const float* c, float*
   if (j < n) rcp[j] = compand_product_exact<T>(c[j]) ? 1.0f / c[j] : 0.0f;
 }
 
+// Bound by VALU issue (71 instructions per value, against 42 us of LDS time in 107 us, over
+// 4096 x 12288 bf16 values with every step on).  What took it to 83.6 us, and 4096 x 4096 from
+// 35.2 to 27: butterfly passes of compile-time stride (LDS offsets become immediates), 16-byte
+// LDS accesses of whole chunks, an unpadded row for the gather, two bf16 roundings per
+// conversion, NaN-keeping v_maximum3 / v_minimum3 clamps, qdq8_values, and one rounding at the
+// end instead of two.
+//
 // One workgroup of NT threads per row of at most 8 NT R values.  R stays at most 4: with
 // 8 chunks per lane the compiler keeps the row in scratch memory instead of registers.
 // With R <= 2 the kernel asks for 8 waves per SIMD (at most 64 VGPRs): two 1024-thread or
@@ -748,7 +824,8 @@ __global__ __launch_bounds__(256) void compand_rcp_kernel(const float* c, float*
 template <typename T, int LV, int R, int NT, bool kGen12, bool kStage = false>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R <= 2 ? 8 : 1))) void act_row_kernel(
     ActRowArgs a) {
-  extern __shared__ float act_row_lds[];
+  extern __shared__ float4 act_row_lds4[];
+  float* const act_row_lds = reinterpret_cast<float*>(act_row_lds4);
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x;
   const T* x = static_cast<const T*>(a.x) + row * a.cols;
@@ -778,11 +855,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R <= 2 ? 8 :
       const int c0 = act_c0<R, NT>(tid, r);
       if (c0 < a.cols) {
         const uint2 sw = *reinterpret_cast<const uint2*>(a.rot_signs + c0);
+        float f[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const int8_t sg = static_cast<int8_t>(((i < 4 ? sw.x : sw.y) >> (8 * (i & 3))) & 0xFFu);
-          act_row_lds[lds_pad(c0) + i] = v[r][i] * static_cast<float>(sg);
+          f[i] = v[r][i] * static_cast<float>(sg);
         }
+        Io<float>::store8(act_row_lds + c0, f);
       }
     }
     __syncthreads();
@@ -795,7 +874,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R <= 2 ? 8 :
         const int pp[8] = {pa.x, pa.y, pa.z, pa.w, pb.x, pb.y, pb.z, pb.w};
 #pragma unroll
         for (int i = 0; i < 8; ++i)  // (one unsigned min keeps any index in range; a valid permutation is)
-          v[r][i] = act_row_lds[lds_pad(static_cast<int>(min(static_cast<uint32_t>(pp[i]), static_cast<uint32_t>(a.cols - 1))))];
+          v[r][i] = act_row_lds[min(static_cast<uint32_t>(pp[i]), static_cast<uint32_t>(a.cols - 1))];
       }
     }
     // every gather has read the row before the transform writes it
@@ -808,18 +887,21 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R <= 2 ? 8 :
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int c0 = act_c0<R, NT>(tid, r);
-    float cs[8];
-    if (a.compand && c0 < a.cols) Io<float>::load8(a.compand + c0, cs);
+    if (a.rot_signs) round8<T>(v[r]);
+    if (a.has_min) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      float t = v[r][i];
-      if (a.rot_signs) t = Io<T>::round(t);
-      if (!__builtin_isnan(t)) {
-        if (a.has_min) t = fmaxf(t, lo);
-        if (a.has_max) t = fminf(t, hi);
-      }
-      if (a.compand && c0 < a.cols) t = Io<T>::round(t * cs[i]);
-      v[r][i] = t;
+      for (int i = 0; i < 8; ++i) v[r][i] = __builtin_elementwise_maximum(v[r][i], lo);
+    }
+    if (a.has_max) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[r][i] = __builtin_elementwise_minimum(v[r][i], hi);
+    }
+    if (a.compand && c0 < a.cols) {
+      float cs[8];
+      Io<float>::load8(a.compand + c0, cs);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[r][i] = v[r][i] * cs[i];
+      round8<T>(v[r]);
     }
   }
   if (a.n) {
@@ -828,9 +910,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R <= 2 ? 8 :
     if constexpr (kGen12) generalized_row<R, NT, RT>(v, act_row_lds, a.cols, a.n, a.div.d, tid);
     else fwht_row<R, NT, RT>(v, act_row_lds, a.cols, a.n, a.div, tid);
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[r][i] = Io<T>::round(v[r][i]);
+    for (int r = 0; r < R; ++r) round8<T>(v[r]);
   }
   // QDQ: every lane takes part (zeros past the row), as qdq8 exchanges values within its 8
   // lanes; then the companding quotient of the quantized values in T: a product with the
@@ -839,27 +919,30 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R <= 2 ? 8 :
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int c0 = act_c0<R, NT>(tid, r);
-    if (a.quant) qdq8<LV>(v[r]);
+    if (a.quant) qdq8_values<LV>(v[r]);
     if (a.compand) {
       float rc[8];
       bool ok = a.compand_rcp != nullptr;
       if (ok && c0 < a.cols) {
         Io<float>::load8(a.compand_rcp + c0, rc);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) ok = ok && rc[i] != 0.0f;
+        // (a zero among them is a zero minimum; reciprocals are never NaN)
+        float least = fminf(fminf(fabsf(rc[0]), fabsf(rc[1])), fabsf(rc[2]));
+        least = fminf(fminf(least, fabsf(rc[3])), fabsf(rc[4]));
+        least = fminf(fminf(least, fabsf(rc[5])), fabsf(rc[6]));
+        ok = fminf(least, fabsf(rc[7])) != 0.0f;
       }
       if (__all(ok)) {
         if (c0 < a.cols)
 #pragma unroll
-          for (int i = 0; i < 8; ++i) v[r][i] = Io<T>::round(in_dtype<T>(v[r][i]) * rc[i]);
+          for (int i = 0; i < 8; ++i) v[r][i] = in_dtype<T>(v[r][i]) * rc[i];
       } else if (c0 < a.cols) {
         float cs[8];
         Io<float>::load8(a.compand + c0, cs);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[r][i] = Io<T>::round(in_dtype<T>(v[r][i]) / cs[i]);
+        for (int i = 0; i < 8; ++i) v[r][i] = in_dtype<T>(v[r][i]) / cs[i];
       }
     }
-    if (c0 < a.cols) Io<T>::store8(y + c0, v[r]);
+    if (c0 < a.cols) Io<T>::store8(y + c0, v[r]);  // the quotient's one rounding to T
   }
 }
 
@@ -988,7 +1071,7 @@ __device__ __forceinline__ void operand_prep_block(const OperandPrepArgs& a, int
         if ((part & 7) == 0) a.pk_meta[pr * 2 + (part >> 3)] = meta;
       }
     } else if (a.quant) {
-      qdq8<LV>(w);
+      qdq8_values<LV>(w);
     }
     if (live && a.y) {
       Io<__hip_bfloat16>::store8(
@@ -1041,7 +1124,7 @@ __device__ __forceinline__ void operand_prep_vt_block(const OperandPrepVtArgs& a
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = Io<Tin>::round(v[i]);
-    if (a.quant) qdq8<LV>(v);
+    if (a.quant) qdq8_values<LV>(v);
     if (a.y && key < a.L)
       Io<__hip_bfloat16>::store8(
           reinterpret_cast<__hip_bfloat16*>(a.y + b * a.yb + h * a.yh + static_cast<int64_t>(key) * a.yl + d0), v);
