@@ -289,51 +289,40 @@ __device__ __forceinline__ void butterfly32_pair(float& x, float& y) {
 }
 
 // HiF4 QDQ of the fragment: 64-value group g (dims 64 g ..) is chunks 4 g .. 4 g + 3 of lanes
-// n and n + 32; the steps of qdq8 (group maximum of the 4-value maxima, E6M2 scale, micro
-// exponents, elements, a NaN anywhere makes the group NaN), with three per-value steps less.
-// The sign of w is copied onto y >= +0: qdq8's `w < 0 ? -y : y` differs only in the sign of a
-// zero that came from w = -0, and a Q value feeds nothing but QK sums that start at +0, which
-// no zero's sign changes.  One unordered comparison tests two values for NaN, and the NaN
-// select runs only when some lane of the wave holds a NaN group.
+// n and n + 32; the steps of qdq8_values (maxima that keep NaN, so that the group maximum's bits
+// tell a NaN group; the NaN select only where some lane of the wave holds one).  The sign of w
+// is copied onto y >= +0: `w < 0 ? -y : y` differs only in the sign of a zero that came from
+// w = -0, and a Q value feeds nothing but QK sums that start at +0, which no zero's sign changes.
 template <int LV>
 __device__ __forceinline__ void q_frag_qdq(float (&v)[8][8]) {
-  int nan_any = 0;
-  int nan_g[2];
+  bool nan_g[2];
 #pragma unroll
   for (int g = 0; g < 2; ++g) {
     float m3a[4], m3b[4];
-    int nan = 0, mx = 0;
+    int mx = 0;
 #pragma unroll
     for (int cc = 0; cc < 4; ++cc) {
       const float* w = v[4 * g + cc];
-      m3a[cc] = fmaxf(fmaxf(fabsf(w[0]), fabsf(w[1])), fmaxf(fabsf(w[2]), fabsf(w[3])));
-      m3b[cc] = fmaxf(fmaxf(fabsf(w[4]), fabsf(w[5])), fmaxf(fabsf(w[6]), fabsf(w[7])));
-#pragma unroll
-      for (int j = 0; j < 8; j += 2) nan |= __builtin_isunordered(w[j], w[j + 1]);
-      mx = max(mx, __float_as_int(fmaxf(m3a[cc], m3b[cc])));
+      m3a[cc] = __builtin_elementwise_maximum(abs_max3_nan(w[0], w[1], w[2]), fabsf(w[3]));
+      m3b[cc] = __builtin_elementwise_maximum(abs_max3_nan(w[4], w[5], w[6]), fabsf(w[7]));
+      mx = max(mx, max(__float_as_int(m3a[cc]), __float_as_int(m3b[cc])));
     }
     mx = max(mx, lane_swap32(mx));
-    nan |= lane_swap32(nan);
-    float sc, rec;
-    hif4_scale<LV>(__int_as_float(mx), sc, rec);
+    nan_g[g] = mx > 0x7F800000;
+    const PQuant q = pquant_setup<LV>(__int_as_float(mx));
 #pragma unroll
     for (int cc = 0; cc < 4; ++cc) {
       float* w = v[4 * g + cc];
-      int ka, kb;
-      hif4_micro<LV>(m3a[cc], m3b[cc], rec, ka, kb);
-      float qa, da, qb, db;
-      hif4_group_mults(sc, rec, ka, qa, da);
-      hif4_group_mults(sc, rec, kb, qb, db);
+      float k4a, k4b;
+      micro_k4<LV>(m3a[cc], m3b[cc], q.rec4, k4a, k4b);
+      const float qa = q.rec4 * inv_k_of(k4a), qb = q.rec4 * inv_k_of(k4b);
+      const float da = k4a * q.s16, db = k4b * q.s16;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float y = hif4_element(fabsf(w[j]), j < 4 ? qa : qb, j < 4 ? da : db);
-        w[j] = __builtin_copysignf(y, w[j]);
-      }
+      for (int j = 0; j < 8; ++j)
+        w[j] = __builtin_copysignf(hif4_element(fabsf(w[j]), j < 4 ? qa : qb, j < 4 ? da : db), w[j]);
     }
-    nan_g[g] = nan;
-    nan_any |= nan;
   }
-  if (__builtin_amdgcn_ballot_w64(nan_any != 0) != 0) {
+  if (__builtin_amdgcn_ballot_w64(nan_g[0] || nan_g[1]) != 0) {
 #pragma unroll
     for (int c = 0; c < 8; ++c)
 #pragma unroll

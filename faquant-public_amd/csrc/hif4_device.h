@@ -181,6 +181,28 @@ __device__ __forceinline__ float k4_of(float x, float e) { return __builtin_amdg
 // 2^-k = (127 - k) << 23 = (256 << 23) - ((129 + k) << 23).
 __device__ __forceinline__ float inv_k_of(float k4) { return __uint_as_float(0x80000000u - __float_as_uint(k4)); }
 
+// NaN-propagating maximum of three magnitudes (one v_maximum3_f32).
+__device__ __forceinline__ float abs_max3_nan(float a, float b, float c) {
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(a), fabsf(b)), fabsf(c));
+}
+
+// 4K of the two 4-value groups of one 8-value group (K = 2^k, k = lv2 + lv3; hif4_micro's rule by
+// exponent masks and med3) from their magnitude maxima.
+template <int LV>
+__device__ __forceinline__ void micro_k4(float m3a, float m3b, float rec4, float& k4a, float& k4b) {
+  const float xa = floor2(m3a * rec4), xb = floor2(m3b * rec4);  // floor2 of 4 t3, t3 = RN(m3 rec)
+  if (LV == 123) {
+    const float e2 = __builtin_amdgcn_fmed3f(fmaxf(xa, xb) * 0.5f, 4.0f, 8.0f);
+    k4a = k4_of(xa, e2);
+    k4b = k4_of(xb, e2);
+  } else if (LV == 12) {
+    k4a = k4b = __builtin_amdgcn_fmed3f(fmaxf(xa, xb), 4.0f, 8.0f);
+  } else {
+    k4a = __builtin_amdgcn_fmed3f(xa, 4.0f, 8.0f);
+    k4b = __builtin_amdgcn_fmed3f(xb, 4.0f, 8.0f);
+  }
+}
+
 // In-register butterfly stage of stride S (1, 2 or 4) on 8 consecutive values: each pair
 // (i, i + S) becomes (left + right, left - right), the order of rotation.py:21-28.
 template <int S>

@@ -175,11 +175,6 @@ __device__ __forceinline__ float group_max8(float v) {
   return __int_as_float(u);
 }
 
-// NaN-propagating maximum of three magnitudes (one v_maximum3_f32).
-__device__ __forceinline__ float abs_max3_nan(float a, float b, float c) {
-  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(a), fabsf(b)), fabsf(c));
-}
-
 // qdq8 without metadata outputs, the same values in fewer instructions (all callers of this
 // form are bound by VALU issue): the maxima propagate NaN, so the group maximum itself says
 // whether the group holds one (a positive NaN's bits are above every number's in the integer
@@ -193,19 +188,8 @@ __device__ __forceinline__ void qdq8_values(float* v) {
   const float m3b = __builtin_elementwise_maximum(abs_max3_nan(v[4], v[5], v[6]), fabsf(v[7]));
   const float m1 = group_max8(__builtin_elementwise_maximum(m3a, m3b));
   const PQuant q = pquant_setup<LV>(m1);
-  // floor2 of 4 t3, t3 = RN(m3 rec)
-  const float xa = floor2(m3a * q.rec4), xb = floor2(m3b * q.rec4);
   float k4a, k4b;
-  if (LV == 123) {
-    const float e2 = __builtin_amdgcn_fmed3f(fmaxf(xa, xb) * 0.5f, 4.0f, 8.0f);
-    k4a = k4_of(xa, e2);
-    k4b = k4_of(xb, e2);
-  } else if (LV == 12) {
-    k4a = k4b = __builtin_amdgcn_fmed3f(fmaxf(xa, xb), 4.0f, 8.0f);
-  } else {
-    k4a = __builtin_amdgcn_fmed3f(xa, 4.0f, 8.0f);
-    k4b = __builtin_amdgcn_fmed3f(xb, 4.0f, 8.0f);
-  }
+  micro_k4<LV>(m3a, m3b, q.rec4, k4a, k4b);
   const float qa = q.rec4 * inv_k_of(k4a), qb = q.rec4 * inv_k_of(k4b);  // 4 rec 2^-k
   const float da = k4a * q.s16, db = k4b * q.s16;                          // s 2^k / 4
 #pragma unroll
