@@ -317,14 +317,14 @@ void launch_attention(const faq::AttnArgs& a, int quant_p, int p_levels, int nor
 // (one wave per SIMD takes 0.6 of two waves' time per tile, and a CU's pair is a long and a
 // short item) and where items are short (one workgroup's setup and epilogue run under the
 // other's tiles).  Measured on 256 CUs, eight against four waves, us:
-//   causal, up to 1.4 items per CU: 32/8 heads 1024 tokens 47.5 / 35.1, 2048 80.3 / 62.4, 2600
-//     99.8 / 86.8, 512 of 8704 keys 284 / 206; just above: 3400 tokens 125 / 127, 4096 164 / 170
-//   causal, many short items: 16 x 512 107 / 99, 8 x 700 81.4 / 77.0; 16 x 1024 269 / 270;
-//     long ones: 8192 tokens 604 / 627
-//   key ranges (items of unequal length): 4 x 1000 64.5 / 53.1, 8 x 1500 193 / 182, 4 x 8000
-//     1552 / 1536; 2 x 16000 3927 / 4084
-//   not causal: 40 heads, 5000 of 640 keys 134 / 131, 20000 of 257 346 / 336; of 2048 240 / 244;
-//     one equal item per CU at most: 1500 tokens 67.3 / 68.8
+//   causal, up to 1.4 items per CU: 32/8 heads 1024 tokens 46.9 / 34.5, 2048 79.7 / 60.3, 2600
+//     99.8 / 88.5, 512 of 8704 keys 284 / 204; just above: 3400 tokens 127 / 129, 4096 166 / 173
+//   causal, many short items: 16 x 512 93.4 / 91.2, 8 x 700 78.7 / 75.5; 16 x 1024 255 / 256;
+//     long ones: 8192 tokens 602 / 629
+//   key ranges (items of unequal length): 4 x 1000 62.0 / 51.4, 8 x 1500 185 / 176, 4 x 8000
+//     1535 / 1529; 2 x 16000 4028 / 4197
+//   not causal: 40 heads, 5000 of 640 keys 132 / 130, 20000 of 257 332 / 320; of 2048 1028 / 1051;
+//     one equal item per CU at most: 1500 tokens 67.4 / 69.0
 bool four_waves(const faq::AttnArgs& a, int64_t n_items) {
   if (a.diag || a.p_dump || a.amask || a.softcap > 0.0f) return false;  // eight-wave forms only
   const char* env = std::getenv("FAQ_ATTN_WAVES");  // test hook: 4 or 8
@@ -594,8 +594,8 @@ int faq_act_prep_rows(const void* x, void* y, int64_t rows, int64_t cols, int dt
   a.rot_perm = o.rot_perm;
   a.rot_block = o.rot_block;
   a.rot_div = sqrt_div(o.rot_block);
-  a.has_min = o.has_min != 0;
-  a.has_max = o.has_max != 0;
+  a.has_min = o.has_min != 0 && o.act_min == o.act_min;  // a NaN bound bounds nothing
+  a.has_max = o.has_max != 0 && o.act_max == o.act_max;
   a.act_min = o.act_min;
   a.act_max = o.act_max;
   a.compand = o.compand;

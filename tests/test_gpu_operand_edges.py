@@ -50,3 +50,13 @@ def test_operand_quantizer_edges(dev, levels, dtype):
     for got in (rows, vt, act):
         assert np.array_equal(np.isnan(got), nan)
         assert np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
+
+
+@pytest.mark.parametrize("bounds", [(float("nan"), 1.0), (-1.0, float("nan")), (float("nan"), float("nan"))])
+def test_a_nan_clamp_bound_bounds_nothing(dev, bounds):
+    from faquant_amd import _ops
+
+    x = torch.randn((5, 256), generator=torch.Generator().manual_seed(3)).to(dev, torch.bfloat16)
+    lo, hi = bounds
+    want = _ops.act_prep_rows(x, levels="123", act_min=None if lo != lo else lo, act_max=None if hi != hi else hi)
+    assert torch.equal(_ops.act_prep_rows(x, levels="123", act_min=lo, act_max=hi), want)
