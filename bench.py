@@ -40,11 +40,11 @@ KERNEL_SOURCES = ("faquant-public_amd/csrc/hif4_attention.hip", "faquant-public_
                   "faquant-public_amd/csrc/hif4_device.h")
 MEASURED_TRAFFIC = {
     # config: (bytes per launch, kernel source sha256 prefix, profile)
-    "qwen8b_32k": (1.675e9, "00a76ba3d16761b7", "profiles/attn_fwd_qwen8b_32k_counters.md"),
-    "qwen8b_8k": (2.159e8, "00a76ba3d16761b7", "profiles/attn_fwd_qwen8b_8k_kernel_trace.md"),
-    "qwen32b_16k": (1.099e9, "00a76ba3d16761b7", "profiles/attn_fwd_qwen32b_16k_kernel_trace.md"),
-    "wan480p": (3.367e9, "00a76ba3d16761b7", "profiles/attn_fwd_wan480p_kernel_trace.md"),
-    "wan720p": (1.873e10, "00a76ba3d16761b7", "profiles/attn_fwd_wan720p_kernel_trace.md"),
+    "qwen8b_32k": (1.672e9, "eb8d50762c34f7d7", "profiles/attn_fwd_qwen8b_32k_counters.md"),
+    "qwen8b_8k": (2.147e8, "eb8d50762c34f7d7", "profiles/attn_fwd_qwen8b_8k_kernel_trace.md"),
+    "qwen32b_16k": (1.101e9, "eb8d50762c34f7d7", "profiles/attn_fwd_qwen32b_16k_kernel_trace.md"),
+    "wan480p": (3.367e9, "eb8d50762c34f7d7", "profiles/attn_fwd_wan480p_kernel_trace.md"),
+    "wan720p": (1.782e10, "eb8d50762c34f7d7", "profiles/attn_fwd_wan720p_kernel_trace.md"),
 }
 
 
