@@ -11,8 +11,9 @@ Reference: src/faquant/wan22_attention.py.  Same public names and signatures:
 accepted and ignored.  P is quantized with the three-level format, as the
 reference kernel's in-register quantizer is.
 
-``make_flash_attention`` fuses rotation, Q/K/V QDQ and attention into three HIP launches
-(K, V, and the attention, which prepares bf16 Q rows as it loads them) when ``input_qdq`` comes from ``faquant_qdq`` (it carries its levels);
+``make_flash_attention`` fuses rotation, Q/K/V QDQ and attention into two HIP launches
+(K and V, and the attention, which prepares bf16 Q rows as it loads them) when ``input_qdq``
+comes from ``faquant_qdq`` (it carries its levels);
 any other callable is applied as given between the rotation and the kernel.
 
 ``patch_attention_modules(model_module, collector)`` (:231-270) installs the same
@@ -141,9 +142,15 @@ def make_flash_attention(
             else:
                 qh, _ = _ops.operand_prep(qh, levels=input_qdq.levels, hadamard=rot, smooth=smooth,
                                           round_dtype=torch.bfloat16)
-            kh, _ = _ops.operand_prep(_as_bhld(k), levels=input_qdq.levels, hadamard=rot, smooth=smooth,
-                                      smooth_divide=True, round_dtype=torch.bfloat16)
-            vt = _ops.operand_prep_vt(_as_bhld(v.to(dtype)), levels=input_qdq.levels)
+            # K and V^T in one launch for bf16
+            kr, vr = _as_bhld(k), _as_bhld(v.to(dtype))
+            kh = torch.empty(kr.shape, device=kr.device, dtype=torch.bfloat16)
+            vt = torch.empty((*vr.shape[:2], vr.shape[3], _ops._pad_keys(vr.shape[2])), device=vr.device,
+                             dtype=torch.bfloat16)
+            _ops.operand_prep_jobs([
+                _ops.prep_job(kr, levels=input_qdq.levels, out=kh, hadamard=rot, smooth=smooth, smooth_divide=True,
+                              round_dtype=torch.bfloat16),
+                _ops.prep_job(vr, levels=input_qdq.levels, vt=vt)], kr.device)
         else:
             if qk_rotation:
                 q, k = rotate_heads(q), rotate_heads(k)
